@@ -539,6 +539,56 @@ bool gemv_requested(int64_t m, int64_t k, const int64_t* ns, int ngroups) {
 
 
 
+// GLU launches of few token rows (no LoRA terms; one shape and statistics kind, as the caller
+// checks): the GEMV's or the small-M kernel's GLU form, or (too many rows, LoRA, a forced MFMA
+// plan) the MFMA kernels.
+struct GluSmallM {
+    enum Kernel { kMfma, kGemv, kSkinny } kernel = kMfma;
+    int row_tiles = 0;  // small-M kernel: row tiles per work-group, half of them gate's
+};
+GluSmallM glu_small_m(int64_t m, int64_t k, int64_t n, bool lora) {
+    GluSmallM r;
+    if (lora || m < 1 || m > kSkinnyMaxM) return r;
+    const char* forced = std::getenv("DECIK_FWD_PLAN");
+    if (forced != nullptr && *forced != 0) return r;
+    // One row: the GEMV on every shape measured. Two rows: its second dot product costs in
+    // proportion to the weight (as in gemv_requested). Graph-replayed at two rows, GEMV against
+    // small-M kernel, us: [4864, 896] 7.0 against 7.2, 1.5B 10.8 against 11.5, [11008, 2048] 13.4
+    // against 15.0; 7B 32.8 against 28.7, [13824, 5120] 34-36 against 32.0. From 3 rows the
+    // small-M kernel wins on every shape (1.5B 14.7 against 11.9).
+    const char* v = std::getenv("DECIK_SMALL_M");
+    const bool gemv_forced = v != nullptr && std::string(v) == "gemv";
+    const bool skinny_forced = v != nullptr && std::string(v) == "skinny";
+    if (!skinny_forced && gemv_glu_fits(m, k) && (m == 1 || gemv_forced || n * k < (int64_t(1) << 25))) {
+        r.kernel = GluSmallM::kGemv;
+        return r;
+    }
+    // The small-M kernel's work-groups take 8 * row_tiles rows of both weights; a CU works off its
+    // share of them: the row tiles with the fewest rows on the busiest CU. Ties go to 4 tiles up to
+    // 16 token rows (two work-groups fit a CU, one's loads behind the other's sums: [13824, 5120]
+    // at 16 rows 39.3 us against 42.8 for 8 tiles and 47.2 for 2), then to the larger.
+    // Graph-replayed at 16 rows, us for 2 / 4 / 6 / 8 / 10 tiles: 7B 39.9 / 37.0 / 39.8 / 47.1 /
+    // 32.7 (80 rows at 2 and 10), 1.5B 14.3 / 14.6 / 13.2 / 15.5 / 18.4 (48 at 2 and 6).
+    const int64_t cus = num_cus();
+    int64_t rows = INT64_MAX;
+    for (int rt : {2, 6, 8, 10, 4}) {
+        if (m > 16 && rt != 4 && rt != 6) continue;
+        const int64_t wgs = (n + 8 * rt - 1) / (8 * rt), per_cu = (wgs + cus - 1) / cus * 8 * rt;
+        const bool tie = m <= 16 || rt > r.row_tiles;
+        if (per_cu < rows || (per_cu == rows && tie)) {
+            rows = per_cu;
+            r.row_tiles = rt;
+        }
+    }
+    // MFMA tiles take 128 rows of both weights a CU in about the time the small-M kernel takes for
+    // 135 of them up to 16 token rows and 117 past (7B: 54.3 us for 128, 32.7 for 80, 44.4-48.9
+    // for 96).
+    const int64_t mfma_rows = ((n + 127) / 128 + cus - 1) / cus * 128;
+    if (rows * (m <= 16 ? 95 : 110) > mfma_rows * 100) return r;
+    r.kernel = GluSmallM::kSkinny;
+    return r;
+}
+
 }  // namespace
 
 int device_cus() { return num_cus(); }
@@ -659,6 +709,15 @@ int dk_nf4_linear_plan(int backward, int64_t m, int64_t k, const int64_t* ns, in
     } else if (small_m_forward(m, glu, lora, ns, ngroups)) {
         p = plan_skinny(m, k, ns, ngroups, single);
         kernel = 5;  // nf4_skinny_kernel
+    } else if (const GluSmallM gs = glu && ngroups == 2 && ns[0] == ns[1] && blocksize >= 64 && k % 64 == 0
+                                        ? glu_small_m(m, k, ns[0], lora)
+                                        : GluSmallM{};
+               gs.kernel != GluSmallM::kMfma) {
+        p = GemmPlan{};
+        p.mt = gs.kernel == GluSmallM::kSkinny ? (m <= 16 ? 1 : 2) : 0;
+        p.waves = 8;
+        p.splits = 1;
+        kernel = gs.kernel == GluSmallM::kGemv ? 4 : 5;
     } else {
         p = plan_fwd(m, k, ns, ngroups, glu, k % 64 == 0 && k % blocksize == 0, single, 1,
                      !(glu && (flags & DK_PLAN_NESTED) != 0));
@@ -808,6 +867,25 @@ static int linear_fwd_impl(const std::string& name, const uint16_t* x, int64_t m
         for (int g = 0; g < ngroups; ++g)
             r.o[g] = ReduceOut{groups[g].y, groups[g].ldy, a.g[g].bias, a.g[g].col_begin, (int32_t)ns[g]};
         return check_hip(launch_splitk_reduce(r, st), "dk_nf4_linear_fwd split-K reduction");
+    }
+    if (const GluSmallM gs = glu ? glu_small_m(m, k, ns[0], any_lora) : GluSmallM{}; gs.kernel != GluSmallM::kMfma) {
+        a.x = reinterpret_cast<const _Float16*>(x);
+        a.ldx = ldx;
+        a.x_bytes = (uint32_t)(((m - 1) * ldx + k) * 2);
+        a.m = (int)m;
+        a.k = (int)k;
+        a.ngroups = 2;
+        a.nested = nested;
+        a.glu = 1;
+        a.h = reinterpret_cast<_Float16*>(h);
+        a.ldh = ldh;
+        const hipStream_t st = static_cast<hipStream_t>(stream);
+        if (gs.kernel == GluSmallM::kGemv) return check_hip(launch_gemv_glu(a, st), "dk_nf4_glu_fwd GEMV launch");
+        a.splits = 1;
+        a.ksteps = a.ksteps_per_split = (int)((k + kSkinnyStep - 1) / kSkinnyStep);
+        const int64_t grid = (ns[0] + 8 * gs.row_tiles - 1) / (8 * gs.row_tiles);
+        if (grid > INT32_MAX / 2) return fail(name + ": problem too large");
+        return check_hip(launch_skinny_glu(a, gs.row_tiles, (int)grid, st), "dk_nf4_glu_fwd small-M launch");
     }
     bool fwd8_ok = k % 64 == 0;
     for (int g = 0; g < ngroups; ++g) fwd8_ok = fwd8_ok && k % groups[g].w.blocksize == 0;

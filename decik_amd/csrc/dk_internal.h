@@ -160,6 +160,11 @@ constexpr int kGemvMaxM = 8;
 // m token rows at this contraction length.
 hipError_t launch_gemv(FwdArgs& a, hipStream_t s);
 bool gemv_fits(int64_t m, int64_t k);
+// the GLU form (a.glu, groups gate and up, a.h; one or two token rows): eight-wave work-groups,
+// one half per weight
+constexpr int kGemvGluMaxM = 2;
+hipError_t launch_gemv_glu(const FwdArgs& a, hipStream_t s);
+bool gemv_glu_fits(int64_t m, int64_t k);
 // CUs of the current device (256 where no device answers)
 int device_cus();
 // waves per work-group of a GEMV launch (k must fit: gemv_fits)
@@ -170,6 +175,9 @@ int gemv_waves(int64_t m, int64_t k, int64_t nrows);
 // each group's first row group. splits > 1: fp32 partial slabs, then splitk_reduce_kernel.
 constexpr int kSkinnyMaxM = 32;
 hipError_t launch_skinny(const FwdArgs& a, int row_tiles, int grid, hipStream_t s);
+// the GLU form: grid work-groups of 8 * row_tiles rows of gate and of up (row_tiles 2, 4,
+// 6, 8 or 10; past 16 token rows 4 or 6), no split
+hipError_t launch_skinny_glu(const FwdArgs& a, int row_tiles, int grid, hipStream_t s);
 // 8-wave forward kernel (32 weight rows x 32*mb tokens per wave), mb = 8 or 9
 hipError_t launch_fwd8(const FwdArgs& a, int mb, int grid, hipStream_t s);
 // 8-wave input-gradient kernel (32 output columns x 32*mb tokens per wave), mb = 2, 4, 7 or 8;

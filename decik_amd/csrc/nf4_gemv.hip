@@ -25,6 +25,15 @@
 //   gives the same bits.
 // - Dequantization as in the other kernels: byte-pair code book in LDS (one 8-byte read per
 //   packed byte), fp32 multiply by the block scale, one fp16 rounding: the reference's bits.
+// - GLU (gate and up with SwiGLU, one or two token rows): a work-group of eight waves takes the
+//   same rows of both weights, waves 0..3 of gate and 4..7 of up, on one staged X; whoever sums
+//   a row sums it of both and writes h = fp16(silu(gate) up). Each half works as a four-wave
+//   work-group does, so gate and up have the bits of the grouped launch. Bound like the plain
+//   form by the latency of a work-group's phases. Before, the MLP of a decode step ran gate and
+//   up on 64-token MFMA tiles (148 work-groups of 56 steps): 7B at one token 57.1 -> 28.2 us
+//   (70 MB, 2.5 TB/s), 1.5B 25.8 -> 9.2.
+#include <type_traits>
+
 #include "dk_internal.h"
 
 namespace dk {
@@ -34,9 +43,10 @@ constexpr int kGemvMaxChunks = 8;  // chunks (16-byte loads) per thread
 constexpr size_t kGemvWideLds = 40 * 1024;  // LDS per work-group past which it takes eight waves
 
 // LDS bytes of a launch: code book, X of the token rows, the chunk partial sums
-static size_t gemv_smem_bytes(int mt, int k, int chunks) {
-    // dynamic part: nested code2 table (256 floats), X, sums (the code book is static)
-    return 256 * sizeof(float) + (size_t)mt * k * 2 + (size_t)mt * chunks * sizeof(float);
+static size_t gemv_smem_bytes(int mt, int k, int chunks, int weights = 1) {
+    // dynamic part: nested code2 tables (256 floats each), X, sums (the code books are static);
+    // chunks: of one weight
+    return weights * 256 * sizeof(float) + (size_t)mt * k * 2 + (size_t)weights * mt * chunks * sizeof(float);
 }
 
 // x plus the x of the lane that DPP control CTRL names (all rows and banks, no bound control)
@@ -55,32 +65,39 @@ __device__ __forceinline__ float row16_sum(float v) {
     return dpp_add<0x128>(v);  // row_ror:8
 }
 
-template <int MT, bool NESTED, int CPT, int TH>
+template <int MT, bool NESTED, int CPT, int TH, bool GLU>
 __global__ __launch_bounds__(TH) void nf4_gemv_kernel(const FwdArgs a, const int rows_per_wg, const uint32_t cpr_inv,
                                                        const int tg_shift) {
-    // byte-pair code book (static: its address is a constant the LDS reads take as an offset)
-    __shared__ float2_t lut2[256];
+    constexpr int NW = GLU ? 2 : 1;   // weights of a work-group
+    constexpr int HT = TH / NW;       // threads per weight
+    // byte-pair code books (static: their addresses are constants the LDS reads take as offsets)
+    __shared__ float2_t lut2[NW * 256];
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    float* c2 = (float*)smem;                        // nested: code2 table
-    _Float16* xs = (_Float16*)(smem + 256 * 4);      // [MT][k], transposed 16-byte pieces
+    float* c2 = (float*)smem;                        // nested: code2 tables
+    _Float16* xs = (_Float16*)(smem + NW * 256 * 4);  // [MT][k], transposed 16-byte pieces
     // token groups: with tg_shift = 1, work-groups 2 b and 2 b + 1 take the same weight rows for
     // token rows 0..MT-1 and MT..2 MT-1 (X of MT rows per work-group)
     const int tg = (int)blockIdx.x & ((1 << tg_shift) - 1);
     const int bid = (int)blockIdx.x >> tg_shift;
     const int K = a.k, M = min(MT, a.m - MT * tg);
     const _Float16* const xg = a.x + (int64_t)(MT * tg) * a.ldx;
-    float* part = (float*)(xs + MT * K);             // [MT][rows * cpr]
+    float* part = (float*)(xs + MT * K);             // [NW][MT][rows * cpr]
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS bases stay scalar
-    int gi = 0;
+    // GLU: waves 0..3 stream the gate rows, waves 4..7 the same rows of up
+    const int sel = GLU ? wave >> 2 : 0;
+    const int ht = GLU ? tid & (HT - 1) : tid;       // thread within its weight's half
+    int gi = sel;
+    if constexpr (!GLU) {
 #pragma unroll
-    for (int q = 1; q < kMaxGroups; ++q)
-        if (q < a.ngroups && bid >= a.g[q].tile_begin) gi = q;
+        for (int q = 1; q < kMaxGroups; ++q)
+            if (q < a.ngroups && bid >= a.g[q].tile_begin) gi = q;
+    }
     const FwdGroupDev& G = a.g[gi];
     const NF4Dev& W = G.w;
     const int N = (int)W.n;
-    const int n0 = (bid - G.tile_begin) * rows_per_wg;
+    const int n0 = (GLU ? bid : bid - G.tile_begin) * rows_per_wg;
     const int rows = min(rows_per_wg, N - n0);
     const int cpr = K >> 5;                 // chunks per row
     const int nch = rows * cpr;             // chunks of this work-group
@@ -99,7 +116,7 @@ __global__ __launch_bounds__(TH) void nf4_gemv_kernel(const FwdArgs a, const int
     uint32_t q8[CPT];
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-        const int c = tid + TH * i;
+        const int c = ht + HT * i;
         const bool ok = c < nch;
         const uint32_t ch = c0 + (uint32_t)c;
         p[i] = bload128(wrs, off_if(ok, ch * 16u));
@@ -133,22 +150,26 @@ __global__ __launch_bounds__(TH) void nf4_gemv_kernel(const FwdArgs a, const int
     // code book and nested code2 table; the barrier (without the release fence of
     // __syncthreads) then publishes every wave's share of them and of X
     wait_vmcnt<0>();
-    if (tid < 256) {
-        lut2[tid] = float2_t{b_hi, b_lo};
-        if constexpr (NESTED) c2[tid] = c2v;
+    if (ht < 256) {
+        lut2[256 * sel + ht] = float2_t{b_hi, b_lo};
+        if constexpr (NESTED) c2[256 * sel + ht] = c2v;
     }
     lds_barrier();
 
-    // k-range p (chunk within its row) of the thread's chunk i: advanced by 256 chunks a step
-    // tid % cpr and TH % cpr without a division: cpr_inv = ceil(2^20 / cpr), exact for
+    // k-range p (chunk within its row) of the thread's chunk i: advanced by HT chunks a step
+    // ht % cpr and HT % cpr without a division: cpr_inv = ceil(2^20 / cpr), exact for
     // numerators below 512 while cpr <= 2048 (the error term n (cpr_inv cpr - 2^20) stays below 2^20)
-    int pk = tid - (int)__umul24((uint32_t)cpr, __umul24((uint32_t)tid, cpr_inv) >> 20);
-    const int dp = TH - cpr * (int)(((uint32_t)TH * cpr_inv) >> 20);
+    int pk = ht - (int)__umul24((uint32_t)cpr, __umul24((uint32_t)ht, cpr_inv) >> 20);
+    const int dp = HT - cpr * (int)(((uint32_t)HT * cpr_inv) >> 20);
+    // the half's dot products; BOOK: the byte offset of its code book, a constant in each copy
+    auto dot_chunks = [&](auto BOOK) __attribute__((always_inline)) {
+    const float* const c2h = c2 + 256 * sel;
+    float* const ph = part + sel * MT * nch;
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-        const int c = tid + TH * i;
+        const int c = ht + HT * i;
         float sc = s[i];
-        if constexpr (NESTED) sc = c2[q8[i]] * sc + offset;  // two roundings (no contraction)
+        if constexpr (NESTED) sc = c2h[q8[i]] * sc + offset;  // two roundings (no contraction)
         const int pc = c < nch ? pk : 0;
         pk += dp;
         if (pk >= cpr) pk -= cpr;
@@ -175,7 +196,7 @@ __global__ __launch_bounds__(TH) void nf4_gemv_kernel(const FwdArgs a, const int
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 // packed byte 4 e + q: weights 32 p + 8 e + 2 q (high nibble) and + 1
-                const float2_t cv = *(const float2_t*)((const char*)lut2 + byte_x8(w, q));
+                const float2_t cv = *(const float2_t*)((const char*)lut2 + BOOK.value + byte_x8(w, q));
                 const half2_t w2 = __builtin_bit_cast(half2_t, pack_half2(cv.x * sc, cv.y * sc));
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
@@ -190,8 +211,11 @@ __global__ __launch_bounds__(TH) void nf4_gemv_kernel(const FwdArgs a, const int
         // their arithmetic below everything and holds every chunk's operands meanwhile)
         if (c < nch)
 #pragma unroll
-            for (int m = 0; m < MT; ++m) part[m * nch + c] = acc[m];
+            for (int m = 0; m < MT; ++m) ph[m * nch + c] = acc[m];
     }
+    };
+    if (sel == 0) dot_chunks(std::integral_constant<int, 0>{});
+    else dot_chunks(std::integral_constant<int, GLU ? 2048 : 0>{});
     lds_barrier();
 
     // each row's sum in a fixed order: a wave sums four rows at once, 16 lanes each; lane j of a
@@ -201,31 +225,48 @@ __global__ __launch_bounds__(TH) void nf4_gemv_kernel(const FwdArgs a, const int
     const int sub = lane >> 4, j16 = lane & 15;
     for (int r0 = 4 * wave; r0 < rows; r0 += TH / 16) {
         const int r = r0 + sub;
-        float v[MT];
+        float v[NW][MT];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            v[m] = 0.0f;
-            if (r < rows) {
-                // four reads in flight at a time, added in slot order
-                const float* pr = part + m * nch + r * cpr;
-                int q = j16;
-                for (; q + 48 < cpr; q += 64) {
-                    const float t0 = pr[q], t1 = pr[q + 16], t2 = pr[q + 32], t3 = pr[q + 48];
-                    v[m] += t0;
-                    v[m] += t1;
-                    v[m] += t2;
-                    v[m] += t3;
+        for (int w = 0; w < NW; ++w)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                float t = 0.0f;
+                if (r < rows) {
+                    // four reads in flight at a time, added in slot order
+                    const float* pr = part + (w * MT + m) * nch + r * cpr;
+                    int q = j16;
+                    for (; q + 48 < cpr; q += 64) {
+                        const float t0 = pr[q], t1 = pr[q + 16], t2 = pr[q + 32], t3 = pr[q + 48];
+                        t += t0;
+                        t += t1;
+                        t += t2;
+                        t += t3;
+                    }
+                    for (; q < cpr; q += 16) t += pr[q];
                 }
-                for (; q < cpr; q += 16) v[m] += pr[q];
+                v[w][m] = row16_sum(t);
             }
-            v[m] = row16_sum(v[m]);
-        }
         if (j16 == 0 && r < rows) {
             const int n = n0 + r;
-            const float b = G.bias != nullptr ? (float)G.bias[n] : 0.0f;
+            float b[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const _Float16* bias = GLU ? a.g[w].bias : G.bias;
+                b[w] = bias != nullptr ? (float)bias[n] : 0.0f;
+            }
 #pragma unroll
             for (int m = 0; m < MT; ++m)
-                if (m < M) G.y[(int64_t)(MT * tg + m) * G.ldy + n] = to_half(v[m] + b);
+                if (m < M) {
+                    const int64_t row = MT * tg + m;
+                    if constexpr (GLU) {
+                        const uint32_t g = pack_half2(v[0][m] + b[0], 0.0f), u = pack_half2(v[1][m] + b[1], 0.0f);
+                        if (a.g[0].y != nullptr) *(uint16_t*)(a.g[0].y + row * a.g[0].ldy + n) = (uint16_t)g;
+                        if (a.g[1].y != nullptr) *(uint16_t*)(a.g[1].y + row * a.g[1].ldy + n) = (uint16_t)u;
+                        *(uint16_t*)(a.h + row * a.ldh + n) = (uint16_t)swiglu_fwd2(g, u);
+                    } else {
+                        G.y[row * G.ldy + n] = to_half(v[0][m] + b[0]);
+                    }
+                }
         }
     }
 }
@@ -331,13 +372,37 @@ static GemvShape gemv_shape(int k, int64_t nrows, int mt, int tgroups) {
     return pick;
 }
 
-template <int MT, bool NESTED, int CPT, int TH>
+// The shape of a GLU launch: 256 threads per weight and the fewest loads per thread (75% filled,
+// where that is possible) that give 4 rows of each weight per token row, so that X, staged once
+// for both weights, costs half their bytes. Graph-replayed at one token, us by loads per thread:
+// 7B gate/up 32.3 at 1 (2 rows), 28.2 at 2 (4 rows), 27.0-27.8 at 3-5, 30 at 6-8; 1.5B 9.2 at 1
+// (5 rows), 9.4-12.0 above; [13824, 5120] 40.9 at 1, 28.4 at 2 (3 rows), 28.6 at 3 (4 rows).
+static GemvShape gemv_glu_shape(int k, int mt) {
+    const int cpr = k >> 5;
+    GemvShape pick{0, 0};
+    for (int cpt = 1; cpt <= kGemvMaxChunks; ++cpt) {
+        const int rows = kGemvThreads * cpt / cpr;
+        if (rows < 1) continue;
+        if (gemv_smem_bytes(mt, k, rows * cpr, 2) > 154 * 1024) break;  // + 4 KB of code books
+        if (pick.cpt != 0 && (double)rows * cpr < 0.75 * kGemvThreads * cpt) continue;
+        pick = GemvShape{cpt, rows, 2 * kGemvThreads};
+        if (rows >= 4 * mt) break;
+    }
+    return pick;
+}
+
+bool gemv_glu_fits(int64_t m, int64_t k) {
+    if (m < 1 || m > kGemvGluMaxM || k <= 0 || k % 32 != 0 || k > kGemvThreads * kGemvMaxChunks * 32) return false;
+    return gemv_glu_shape((int)k, gemv_mt(m)).rows >= 1;
+}
+
+template <int MT, bool NESTED, int CPT, int TH, bool GLU = false>
 static hipError_t launch_gemv_th(const FwdArgs& a, int rows, int grid, int tg_shift, hipStream_t s) {
-    const size_t lds = gemv_smem_bytes(MT, a.k, rows * (a.k >> 5));
-    const hipError_t e = allow_dynamic_lds((const void*)nf4_gemv_kernel<MT, NESTED, CPT, TH>, lds);
+    const size_t lds = gemv_smem_bytes(MT, a.k, rows * (a.k >> 5), GLU ? 2 : 1);
+    const hipError_t e = allow_dynamic_lds((const void*)nf4_gemv_kernel<MT, NESTED, CPT, TH, GLU>, lds);
     if (e != hipSuccess) return e;
     const uint32_t cpr = (uint32_t)(a.k >> 5), cpr_inv = ((1u << 20) + cpr - 1) / cpr;
-    hipLaunchKernelGGL((nf4_gemv_kernel<MT, NESTED, CPT, TH>), dim3(grid << tg_shift), dim3(TH), lds, s, a, rows, cpr_inv,
+    hipLaunchKernelGGL((nf4_gemv_kernel<MT, NESTED, CPT, TH, GLU>), dim3(grid << tg_shift), dim3(TH), lds, s, a, rows, cpr_inv,
                        tg_shift);
     return hipGetLastError();
 }
@@ -389,6 +454,27 @@ hipError_t launch_gemv(FwdArgs& a, hipStream_t s) {
         case 2: return a.nested ? launch_gemv_cpt<2, true>(a, sh, grid, 0, s) : launch_gemv_cpt<2, false>(a, sh, grid, 0, s);
         default: return a.nested ? launch_gemv_cpt<4, true>(a, sh, grid, tg_shift, s) : launch_gemv_cpt<4, false>(a, sh, grid, tg_shift, s);
     }
+}
+
+template <int MT, bool NESTED>
+static hipError_t launch_gemv_glu_t(const FwdArgs& a, const GemvShape& sh, int grid, hipStream_t s) {
+    switch (sh.cpt) {
+#define X(C) \
+    case C: return launch_gemv_th<MT, NESTED, C, 2 * kGemvThreads, true>(a, sh.rows, grid, 0, s);
+        X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
+#undef X
+        default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t launch_gemv_glu(const FwdArgs& a, hipStream_t s) {
+    if (!a.glu || a.ngroups != 2 || a.g[0].w.n != a.g[1].w.n || a.h == nullptr || !gemv_glu_fits(a.m, a.k) ||
+        a.g[0].lora_u != nullptr || a.g[1].lora_u != nullptr)
+        return hipErrorInvalidValue;
+    const GemvShape sh = gemv_glu_shape(a.k, gemv_mt(a.m));
+    const int grid = (int)((a.g[0].w.n + sh.rows - 1) / sh.rows);
+    if (a.m == 1) return a.nested ? launch_gemv_glu_t<1, true>(a, sh, grid, s) : launch_gemv_glu_t<1, false>(a, sh, grid, s);
+    return a.nested ? launch_gemv_glu_t<2, true>(a, sh, grid, s) : launch_gemv_glu_t<2, false>(a, sh, grid, s);
 }
 
 }  // namespace dk

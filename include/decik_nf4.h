@@ -163,7 +163,8 @@ int dk_nf4_linear_rope_fwd(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
  * dk_swiglu_fwd. One launch when gate and up have the same statistics kind (both plain or both
  * nested, as bitsandbytes stores them), blocksize >= 64 and k % 64 == 0; then groups[i].y may be
  * NULL (not stored). Other weights run as the grouped launch then the SwiGLU kernel and need both
- * y, with rows contiguous (ldy = ldh = n). No workspace. */
+ * y, with rows contiguous (ldy = ldh = n). Up to 32 token rows without LoRA terms run the GLU forms
+ * of the GEMV and the small-M kernel. No workspace. */
 int dk_nf4_glu_fwd(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
                    const dk_linear_fwd_group* groups, int lora_rank, uint16_t* h, int64_t ldh,
                    void* stream);
@@ -320,9 +321,11 @@ int dk_swiglu_bwd(const uint16_t* grad, const uint16_t* gate, const uint16_t* up
  * earlier input-gradient kernel), 3 nf4_bwd8_kernel, 4 nf4_gemv_kernel (forward launches of one
  * token row, two with fewer than 2^25 weights and k <= 12288 (any k up to 2^24 weights), 3-4
  * with at most 2^24 weights, 5-8 with fewer than 2^23 weights
- * and 8 k <= 32768, without LoRA terms or the GLU epilogue), 5
+ * and 8 k <= 32768, without LoRA terms; GLU launches of one token row, two with fewer than 2^25
+ * weights each), 5
  * nf4_skinny_kernel (such launches of up to 32 token rows otherwise, but past 16 rows not for
- * weights of more 64-row groups than the device has CUs; out[2] is then its contraction splits); DECIK_SMALL_M = gemv / skinny picks one
+ * weights of more 64-row groups than the device has CUs, GLU launches not where its row groups
+ * would outlast the MFMA tiles; out[2] is then its contraction splits); DECIK_SMALL_M = gemv / skinny picks one
  * of the two where both may run). Host-only (no GPU call);
  * honours DECIK_FWD_PLAN / DECIK_BWD_PLAN / DECIK_SMALL_M like the launches. Returns 0, or nonzero
  * with dk_last_error() on bad arguments. */
