@@ -40,13 +40,16 @@
 
 namespace dk {
 
-// LDS transpose read (gfx950 ds_read_b64_tr_b4): the 16 lanes of each lane group read 8 bytes each
-// (row r = lane r's 16 nibbles, low nibble first); lane i of the group receives nibble i of rows
-// 0..15, in order (row e at bits 4 e of the 64-bit result).
-__device__ __forceinline__ u32x2_t lds_tr4(const uint8_t* p) {
-    typedef int v2i __attribute__((ext_vector_type(2)));
-    const v2i r = __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) v2i*)p);
-    return u32x2_t{(uint32_t)r[0], (uint32_t)r[1]};
+// LDS transpose reads (gfx950 ds_read_b64_tr_b4) of one step: the 16 lanes of each lane group read 8
+// bytes each (row r = lane r's 16 nibbles, low nibble first); lane i of the group receives nibble i
+// of rows 0..15, in order (row e at bits 4 e of the 64-bit result). lo: rows 0..15 of the lane
+// group's half step, hi: rows 16..31, 256 bytes on. Written as one asm block with its own wait: the
+// builtin's read counts as aliasing every buffer -> LDS load in flight, so each one drained them all
+// (s_waitcnt vmcnt(0), twice a step).
+__device__ __forceinline__ void lds_tr4x2(const uint8_t* p, u32x2_t& lo, u32x2_t& hi) {
+    const auto l = (__attribute__((address_space(3))) const uint8_t*)p;
+    asm volatile("ds_read_b64_tr_b4 %0, %2\n\tds_read_b64_tr_b4 %1, %2 offset:256\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(lo), "=&v"(hi) : "v"(l) : "memory");
 }
 
 constexpr int kB8Waves = 8;
@@ -352,15 +355,15 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
         scales_3(t0, 0);
 
         half8_t xf[MB], w, wn;
-        u32x2_t tr;      // the last transposed read: this lane's nibbles of two slices
+        u32x2_t tr[2];   // the step's transposed reads: this lane's nibbles of slices 0, 1 and 2, 3
         uint32_t d0;     // next slice: this lane's nibbles of its 8 rows (row e at bits 4 e)
         float4_t s0, s1; // ... their row scales
         float v[8];      // ... their code-book values
         uint32_t e0;     // two-slice pipeline: the nibbles and scales of the slice after
         float4_t t0s, t1s;
-        auto stage_A = [&](int rw, int sidx, int j) __attribute__((always_inline)) {
-            if ((j & 1) == 0) tr = lds_tr4(wring + rw + pkl + 128 * j);
-            const uint32_t dj = (j & 1) ? tr[1] : tr[0];
+        auto fetch_tr = [&](int rw) __attribute__((always_inline)) { lds_tr4x2(wring + rw + pkl, tr[0], tr[1]); };
+        auto stage_A = [&](int sidx, int j) __attribute__((always_inline)) {
+            const uint32_t dj = tr[j >> 1][j & 1];
             const float* sc = stab + 64 * sidx + 32 * g + 8 * j;
             if constexpr (P2) {
                 e0 = dj;
@@ -402,14 +405,15 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
         };
 
         // slice 0 of the first step (and, two slices deep, slice 1's packed dwords and scales)
-        stage_A(rw0, si0, 0);
+        fetch_tr(rw0);
+        stage_A(si0, 0);
         advance();
 #pragma unroll
         for (int i = 0; i < MB; ++i) xf[i] = xfrag(rd0, i, 0);
         stage_B();
         w = stage_C();
         if constexpr (P2) {
-            stage_A(rw0, si0, 1);
+            stage_A(si0, 1);
             advance();
         }
 
@@ -440,10 +444,14 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
                     if (q == 0) {
                         // step t+1's loads (this wave's) landed; its row scales follow in this
                         // slice, before any stage A reads them
-                        if (j == JW) wait_vmcnt<NL>();
                         const int ja = j + LA;  // the slice stage A prepares
-                        if (ja < 4) stage_A(rw0, si0, ja);
-                        else stage_A(rw1, 1 - si0, ja - 4);
+                        if (ja < 4) stage_A(si0, ja);
+                        else stage_A(1 - si0, ja - 4);
+                        if (j == JW) {
+                            // (slice 3's nibbles are out: the transposed reads move on a step)
+                            wait_vmcnt<NL>();
+                            fetch_tr(rw1);
+                        }
                     }
                     if (j == JW) {
                         if (q == qS1) scales_1(rw1);
