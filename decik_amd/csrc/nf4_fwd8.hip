@@ -47,9 +47,13 @@ constexpr int kF8WSlot = 1536;
 // largest of the epilogues; it reuses the X ring, which is sized to hold it.
 constexpr int kF8Stage = 2 * 32 * (256 * 4 + 16);
 
-// bytes of the X ring region: three step buffers, or the epilogue staging if that is larger
+// X ring: three step buffers, four with few token blocks (see the main loop)
+__host__ __device__ constexpr int fwd8_xbufs(int mb) { return mb <= 4 ? 4 : 3; }
+
+// bytes of the X ring region: the step buffers, or the epilogue staging if that is larger
 __host__ __device__ constexpr int fwd8_xring_bytes(int mb) {
-    return 3 * 32 * mb * 128 > kF8Stage ? 3 * 32 * mb * 128 : kF8Stage;
+    const int ring = fwd8_xbufs(mb) * 32 * mb * 128;
+    return ring > kF8Stage ? ring : kF8Stage;
 }
 
 __host__ __device__ constexpr size_t fwd8_smem_bytes(int mb) {
@@ -66,8 +70,13 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     static_assert(XCH % 64 == 0, "a wave's X load is wholly inside or past the tile");
     static_assert(kF8Stage <= fwd8_xring_bytes(MB), "epilogue staging fits the X ring");
     constexpr int NP = XPT + 2;                                  // load parts per step
+    constexpr int SL = NESTED ? 2 : 1;                           // loads of a statistics part
     static_assert(NP <= 8 && MB >= 2, "at most two load parts per slice");
-    constexpr int L3 = spread_loads(NP, NESTED ? 2 : 1, -1);     // loads issued in slice 3
+    // slices ahead of their MFMAs that code-book values and X fragments are read, and with them the
+    // slice that holds the step boundary and the one that fetches the next step's packed weights
+    constexpr int LB = MB <= 4 ? 2 : 1, LX = MB <= 2 ? 2 : 1;
+    constexpr int JB = 4 - LX, JF = 3 - LB;
+    constexpr int XBUFS = fwd8_xbufs(MB);
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     // byte-pair code books (gate, up in GLU mode; the same book otherwise): entry 256 b + byte
     // holds (code_b[byte >> 4], code_b[byte & 15]), the two weights of one packed byte
@@ -210,19 +219,26 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     // every load of step t (the prologue)
     auto load_step = [&](int t, int rx, int rw, bool live) __attribute__((always_inline)) {
 #pragma unroll
-        for (int p = 0; p < XPT + 2; ++p) load_part(p, t, rx, rw, live);
+        for (int i = 0; i < NP; ++i) load_part(spread_part(i, XPT), t, rx, rw, live);
     };
-    // fp32 scale of this lane's row at step t (0 outside the weight)
-    auto scale_of = [&](const uint8_t* slot) __attribute__((always_inline)) -> float {
+    // fp32 scale of this lane's row (0 outside the weight) from its statistics, in three parts: the
+    // slot's values, the code2 lookup, the scale
+    uint32_t sq = 0;
+    float sa = 0.0f, sc2 = 0.0f;
+    auto scale_1 = [&](const uint8_t* slot) __attribute__((always_inline)) {
         const int si = wide ? lane : l32;
-        float sc;
         if constexpr (NESTED) {
-            const uint32_t q = slot[1024 + 4 * si];
-            const float a2 = *(const float*)(slot + 1280 + 4 * si);
-            sc = c2w[q] * a2 + offset;
+            sq = slot[1024 + 4 * si];
+            sa = *(const float*)(slot + 1280 + 4 * si);
         } else {
-            sc = *(const float*)(slot + 1024 + 4 * si);
+            sa = *(const float*)(slot + 1024 + 4 * si);
         }
+    };
+    auto scale_2 = [&]() __attribute__((always_inline)) {
+        if constexpr (NESTED) sc2 = c2w[sq];
+    };
+    auto scale_3 = [&]() __attribute__((always_inline)) -> float {
+        const float sc = NESTED ? sc2 * sa + offset : sa;
         return rowok ? sc : 0.0f;
     };
     auto xfrag = [&](const uint8_t* xb, int i, int j) __attribute__((always_inline)) -> half8_t {
@@ -234,14 +250,18 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     for (int i = 0; i < MB; ++i) acc[i] = float16_t{};
 
     // Ring buffers: step t uses X buffer rx0 (byte offset in the X ring) and weight slot rw0;
-    // step t + 1 uses rx1 / rw1; step t + 3 reuses step t's.
+    // step t + 1 uses rx1 / rw1. Step t + 3 reuses step t's weight slot and X buffer, or with four
+    // X buffers (rx3) step t - 1's.
     int rx0 = 0, rw0 = 0, rx1 = XBUF, rw1 = wslot_bytes, rx2 = 2 * XBUF, rw2 = 2 * wslot_bytes;
-    // Prologue: two steps and the slice-3 parts of the third in flight (issued before the LoRA
+    int rx3 = XBUFS == 4 ? 3 * XBUF : 0;
+    // Prologue: two steps and the first parts of the third in flight (issued before the LoRA
     // term, whose loads then share their round trip); the wait for the first follows the LoRA term.
     load_step(ks0, 0, 0, true);
     load_step(ks0 + 1, XBUF, wslot_bytes, ks0 + 1 < ks1);
 #pragma unroll
-    for (int i = 0; i < NP; i += 4) load_part(spread_part(i, XPT), ks0 + 2, rx2, rw2, ks0 + 2 < ks1);
+    for (int c = 0; c < LX; ++c)
+#pragma unroll
+        for (int i = c; i < NP; i += 4) load_part(spread_part(i, XPT), ks0 + 2, rx2, rw2, ks0 + 2 < ks1);
 
     // LoRA term s * U.B^T first (split 0 only), as in nf4_fwd_kernel, for this wave's weight.
     {
@@ -266,85 +286,99 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     lut2[tid] = float2_t{book_hi, book_lo};
     if constexpr (NESTED)
         if (glu || tid < 256) c2[tid] = c2v;
-    wait_vmcnt<NL + L3>();
+    wait_vmcnt<NL + spread_loads(NP, SL, LX)>();
     lds_barrier();
 
-    u32x4_t p;  // packed weights of the current step (slice j: dword j)
-    float s;    // their scale
+    u32x4_t p;  // packed weights of the step whose code-book values are read next (slice j: dword j)
+    float s;    // the scale of the step that is packed next
     auto fetch_step = [&](int rw) __attribute__((always_inline)) {
         const uint8_t* ws = wring + rw;
         p = *(const u32x4_t*)(ws + 16 * lane);
-        s = scale_of(ws);
+        scale_1(ws);
     };
-    half8_t xf[MB], w, wn;
-    uint32_t pa[4];   // code-book pair addresses of the next slice's 4 packed bytes
-    float v[8];       // its code-book values
-    fetch_step(rw0);
+    half8_t xf[LX][MB], w, wn;
+    uint32_t pa[4];   // code-book pair addresses of a slice's 4 packed bytes
+    float v[LB][8];   // code-book values (slice j: v[j % LB])
+    auto stage_A = [&](uint32_t d) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < MB; ++i) xf[i] = xfrag(xs + rx0, i, 0);
-    {
-        u32x4_t o;
+        for (int e = 0; e < 4; ++e) pa[e] = pair_addr(d, e);
+    };
+    auto stage_B = [&](float* vs) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float2_t cv = pair_at(pair_addr(p[0], e));
-            o[e] = pack_half2(cv.x * s, cv.y * s);
+            const float2_t cv = pair_at(pa[e]);
+            vs[2 * e] = cv.x;
+            vs[2 * e + 1] = cv.y;
         }
-        w = __builtin_bit_cast(half8_t, o);
+    };
+    auto stage_C = [&](const float* vs) __attribute__((always_inline)) -> half8_t {
+        u32x4_t o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = pack_half2(vs[2 * e] * s, vs[2 * e + 1] * s);
+        return __builtin_bit_cast(half8_t, o);
+    };
+    fetch_step(rw0);
+    scale_2();
+    s = scale_3();
+#pragma unroll
+    for (int j = 0; j < LX; ++j)
+#pragma unroll
+        for (int i = 0; i < MB; ++i) xf[j][i] = xfrag(xs + rx0, i, j);
+#pragma unroll
+    for (int j = 0; j < LB; ++j) {
+        stage_A(p[j]);
+        stage_B(v[j]);
     }
-    // stage positions (MFMA index after which a stage runs). With seven or more MFMAs a slice the
-    // stages take separate gaps, and in slice 3, whose first gap holds the step boundary, the
-    // address and code-book stages move one gap later; with fewer (MB = 2, 4) the code-book reads
-    // follow the addresses in the first gap of every slice and the scaling takes the last gap
-    // that leaves them time to land.
-    constexpr bool SMALL = MB < 7;
-    constexpr int qA = 0, qB = SMALL ? 0 : 1, qC = SMALL ? (MB > 2 ? MB - 2 : 1) : MB - 3;
-    constexpr int q3 = SMALL ? 0 : 1;  // slice 3's shift of stages A and B
+    w = stage_C(v[0]);
+    // Stage positions (MFMA index after which a stage runs). Slice j reads the code-book values of
+    // slice j + LB (addresses A, reads B) and packs the weights of slice j + 1 (C). With seven or
+    // more MFMAs a slice that is one slice ahead, the stages in gaps of their own. With fewer
+    // (MB = 2, 4) a slice is over before its LDS reads are back, so code-book values are read two
+    // slices ahead, at MB = 2 X fragments too, and four X buffers (step t + 3 loads into step
+    // t - 1's, whose readers are long done) leave the boundary nothing to drain. (One slice ahead
+    // and draining, a step took about 2100 cycles at MB = 2, twice the LDS's own time.)
+    // The next step's packed weights and statistics, a wave's own, are fetched in slice JF, their
+    // scale follows by slice 3: neither is on the boundary's path.
+    constexpr int qA = 0, qB = MB > 4 ? 1 : 0, qC = MB > 4 ? MB - 3 : (MB > 2 ? 2 : 1);
+    constexpr int jS2 = MB > 4 ? JF : JF + 1, qS2 = MB > 4 ? MB - 3 : 0, qS3 = MB > 4 ? 1 : 0;
+    // loads that may be in flight when step t+1's packed weights and statistics are fetched
+    constexpr int NF = spread_after_stats(NP, SL, LX, JF);
     for (int t = ks0; t < ks1; ++t) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int jn = (j + 1) & 3;
 #pragma unroll
             for (int q = 0; q < MB; ++q) {
-                acc[q] = mfma32x32x16(w, xf[q], acc[q]);
-                if (j == 3 && q == 0) {
-                    // step t+1's loads have landed (only step t+2's may be in flight): fetch this
-                    // wave's packed bytes and scale; after the barrier no wave reads step t's
-                    // slots again: refill them with step t+3. Past the last step these reads
-                    // see stale slots and their values go unused.
+                acc[q] = mfma32x32x16(w, xf[j % LX][q], acc[q]);
+                if (j == JB && q == 0) {
+                    // step t+1's loads have landed (only step t+2's may be in flight); after the
+                    // barrier no wave reads the buffers that step t+3 loads into. Past the last
+                    // step the reads below see stale slots and their values go unused.
                     wait_vmcnt<NL>();
-                    fetch_step(rw1);
-                    lds_barrier();
+                    if constexpr (XBUFS == 4) bare_barrier();
+                    else lds_barrier();
                 }
-                // ring refills: slice 3 starts step t+3 in the slots step t has freed, slices 0-2
-                // continue step t+2
+                // ring refills: from the boundary on step t+3's, before it the rest of step t+2's
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
-                    const int i = 4 * r + (j == 3 ? 0 : j + 1);
+                    const int i = 4 * r + ((j - JB) & 3);
                     if (i < NP && q == r * (MB / 2)) {
-                        if (j == 3) load_part(spread_part(i, XPT), t + 3, rx0, rw0, t + 3 < ks1);
+                        if (j >= JB) load_part(spread_part(i, XPT), t + 3, XBUFS == 4 ? rx3 : rx0, rw0, t + 3 < ks1);
                         else load_part(spread_part(i, XPT), t + 2, rx2, rw2, t + 2 < ks1);
                     }
                 }
-                // refill the X fragment the MFMA above has read (slice j + 1)
-                xf[q] = xfrag(xs + (j < 3 ? rx0 : rx1), q, jn);
-                if (q == (j < 3 ? qA : qA + q3)) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) pa[e] = pair_addr(p[jn], e);
-                }
-                if (q == (j < 3 ? qB : qB + q3)) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float2_t cv = pair_at(pa[e]);
-                        v[2 * e] = cv.x;
-                        v[2 * e + 1] = cv.y;
+                // refill the X fragment the MFMA above has read (slice j + LX)
+                xf[j % LX][q] = xfrag(xs + (j + LX < 4 ? rx0 : rx1), q, (j + LX) & 3);
+                if (q == qA) {
+                    stage_A(p[(j + LB) & 3]);
+                    if (j == JF) {
+                        wait_vmcnt<NF>();
+                        fetch_step(rw1);
                     }
                 }
-                if (q == qC) {
-                    u32x4_t o;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = pack_half2(v[2 * e] * s, v[2 * e + 1] * s);
-                    wn = __builtin_bit_cast(half8_t, o);
-                }
+                if (q == qB) stage_B(v[(j + LB) % LB]);
+                if (j == jS2 && q == qS2) scale_2();
+                if (j == 3 && q == qS3) s = scale_3();
+                if (q == qC) wn = stage_C(v[(j + 1) % LB]);
                 __builtin_amdgcn_sched_barrier(0);
             }
             w = wn;
@@ -355,8 +389,9 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
         rw0 = rw1;
         rx1 = rx2;
         rw1 = rw2;
-        rx2 = rxo;
+        rx2 = XBUFS == 4 ? rx3 : rxo;
         rw2 = rwo;
+        if constexpr (XBUFS == 4) rx3 = rxo;
     }
     wait_vmcnt<0>();
     lds_barrier();  // every wave is done with the X ring: it becomes the staging area
