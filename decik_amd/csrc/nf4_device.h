@@ -93,6 +93,14 @@ __device__ __forceinline__ void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory");
 }
 
+// Wait until at most n of this wave's LDS and scalar-memory operations are outstanding, as an
+// instruction the compiler knows: reads it covers need no waits of their own.
+template <int n>
+__device__ __forceinline__ void wait_lgkmcnt() {
+    static_assert(n >= 0 && n < 16, "lgkmcnt range");
+    __builtin_amdgcn_s_waitcnt(0xC07F | (n << 8));  // vmcnt and expcnt at their maxima: not waited for
+}
+
 // Work-group barrier for LDS hand-offs: this wave's LDS writes complete, then s_barrier. Unlike
 // __syncthreads() it carries no release fence, which would wait for every outstanding global ->
 // LDS load (vmcnt(0)) and so serialize the prefetch; loads the next phase reads are covered by
@@ -125,6 +133,28 @@ __device__ __forceinline__ uint32_t pack_half2(float a, float b) {
     h.x = (_Float16)a;
     h.y = (_Float16)b;
     return __builtin_bit_cast(uint32_t, h);
+}
+
+// Four fp16 pairs of eight products v[e] * s[e]: the products first, then the conversions. Left to
+// itself the compiler alternates them, and a conversion right after its product costs a wait state.
+__device__ __forceinline__ u32x4_t pack_half8(const float* v, const float* s) {
+    float p[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) p[e] = v[e] * s[e];
+    asm("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7]));
+    u32x4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        half2_t h;
+        h.x = (_Float16)p[2 * e];
+        h.y = (_Float16)p[2 * e + 1];
+        o[e] = __builtin_bit_cast(uint32_t, h);
+    }
+    return o;
+}
+__device__ __forceinline__ u32x4_t pack_half8(const float* v, float s) {
+    const float ss[8] = {s, s, s, s, s, s, s, s};
+    return pack_half8(v, ss);
 }
 
 // fp32 -> fp16 (round to nearest even), the value opaque to the compiler (see pack_half2).

@@ -70,13 +70,14 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
 
     // the weights of the work-group (GLU: gate, up; one shape and block size)
     rsrc_t wrs[NW], ars[NW], a2rs[NW];
-    float offset[NW];
+    float offset[NW], c2v[NW], book_hi[NW], book_lo[NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
         const NF4Dev& V = GLU ? a.g[w].w : W;
-        const float* book = V.code;
-        if (tid < 256) lut2[256 * w + tid] = float2_t{book[tid >> 4], book[tid & 15]};
-        if (NESTED && tid >= 256) c2[256 * w + tid - 256] = V.code2[tid - 256];
+        // (written to LDS once the first step's loads are on their way too)
+        book_hi[w] = V.code[(tid >> 4) & 15];
+        book_lo[w] = V.code[tid & 15];
+        if (NESTED && tid < 256) c2v[w] = V.code2[tid];
         offset[w] = NESTED ? *V.offset : 0.0f;
         wrs[w] = make_rsrc(V.packed, V.packed_bytes);
         ars[w] = make_rsrc(NESTED ? (const void*)V.absmax8 : (const void*)V.absmaxf, V.absmax_bytes);
@@ -137,27 +138,44 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
             for (int t = 0; t < 4; ++t)
                 st.x[b][t] = bload128(xrs, off_if(kok && tok[b], (uint32_t)((tok[b] ? 16 * b + i : 0) * ldx + k + 8 * t) * 2u));
     };
-    auto compute = [&](const Step& st) __attribute__((always_inline)) {
+    // Row tile r, MFMA t of a step is item 4 r + t: 8 weights a lane. The code-book values of an item
+    // are read while the one before is packed (the scheduling barriers keep that order: left to
+    // itself the compiler waits for each item's four reads as soon as they are issued), and one wait
+    // covers the four. Two waves a SIMD issue an instruction every 4 to 5 cycles between them, so it
+    // is the instructions per item that count, 34 before and 24 now. 7B at 16 rows: gate and up 28.3
+    // -> 25.3 us, q/k/v 8.7 -> 7.8; reading two items ahead was no faster, nor was a code book with
+    // one copy per pair of LDS banks, which takes the bank conflicts out of every read (26.5 -> 28.2).
+    auto compute = [&](Step& st) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-            const int wi = r / WT;
-            float s = st.s[r];
-            if constexpr (NESTED) s = c2[256 * wi + st.q8[r]] * s + offset[wi];  // two roundings (no contraction)
-            if (!rok[r % WT]) s = 0.0f;
+            const int w = r / WT;
+            if constexpr (NESTED) st.s[r] = c2[256 * w + st.q8[r]] * st.s[r] + offset[w];  // two roundings (no contraction)
+            if (!rok[r % WT]) st.s[r] = 0.0f;
+        }
+        float v[2][8];
+        auto look = [&](int item) __attribute__((always_inline)) {
+            const int r = item / 4;
+            const uint32_t w = st.p[r][item % 4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const uint32_t w = st.p[r][t];
-                u32x4_t o;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float2_t cv = *(const float2_t*)((const char*)lut2 + 2048 * wi + (((w >> (8 * e)) & 0xFFu) << 3));
-                    o[e] = pack_half2(cv.x * s, cv.y * s);
-                }
-                const half8_t av = __builtin_bit_cast(half8_t, o);
-#pragma unroll
-                for (int b = 0; b < MT; ++b)
-                    acc[r][b] = mfma16x16x32(av, __builtin_bit_cast(half8_t, st.x[b][t]), acc[r][b]);
+            for (int e = 0; e < 4; ++e) {
+                const float2_t cv = *(const float2_t*)((const char*)lut2 + 2048 * (r / WT) + byte_x8(w, e));
+                v[item % 2][2 * e] = cv.x;
+                v[item % 2][2 * e + 1] = cv.y;
             }
+        };
+        look(0);
+#pragma unroll
+        for (int item = 0; item < 4 * RT; ++item) {
+            const int r = item / 4, t = item % 4;
+            if (item + 1 < 4 * RT) look(item + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (item + 1 < 4 * RT) wait_lgkmcnt<4>();
+            else wait_lgkmcnt<0>();
+            __builtin_amdgcn_sched_barrier(0);
+            const half8_t av = __builtin_bit_cast(half8_t, pack_half8(v[item % 2], st.s[r]));
+#pragma unroll
+            for (int b = 0; b < MT; ++b)
+                acc[r][b] = mfma16x16x32(av, __builtin_bit_cast(half8_t, st.x[b][t]), acc[r][b]);
         }
     };
 
@@ -169,6 +187,11 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
     Step sa, sb;
     int ss = s0 + wave;
     load(ss, sa);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        if (tid < 256) lut2[256 * w + tid] = float2_t{book_hi[w], book_lo[w]};
+        if (NESTED && tid < 256) c2[256 * w + tid] = c2v[w];
+    }
     __syncthreads();  // the code book in LDS (the first step's loads are already in flight)
     while (ss < s1) {
         load(ss + kSkWaves, sb);
