@@ -65,10 +65,11 @@ constexpr int kB8ScaleBytes = 2 * 64 * 4;  // per wave: row-scale tables of two 
 // Epilogue staging: two 32-token blocks of fp32 tiles (rows 1040 bytes apart), in the dY ring
 // and the weight rings and scale tables behind it; the dY ring region is sized so that it fits.
 constexpr int kB8Stage = 2 * 32 * (kB8BN * 4 + 16);
+// dY ring: three step buffers, four with few token blocks (see the main loop)
+__host__ __device__ constexpr int bwd8_dbufs(int mb) { return mb <= 4 ? 4 : 3; }
 __host__ __device__ constexpr int bwd8_dring_bytes(int mb) {
-    return 3 * 32 * mb * 128 + kB8Waves * (3 * kB8WSlot + kB8ScaleBytes) >= kB8Stage
-               ? 3 * 32 * mb * 128
-               : kB8Stage - kB8Waves * (3 * kB8WSlot + kB8ScaleBytes);
+    const int ring = bwd8_dbufs(mb) * 32 * mb * 128, rest = kB8Waves * (3 * kB8WSlot + kB8ScaleBytes);
+    return ring + rest >= kB8Stage ? ring : kB8Stage - rest;
 }
 
 __host__ __device__ constexpr size_t bwd8_smem_bytes(int mb) {
@@ -137,17 +138,22 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
 #pragma unroll
     for (int i = 0; i < MB; ++i) acc[i] = float16_t{};
 
-    // stage positions (MFMA index after which a stage runs). With few MFMAs per slice (P2) the
-    // packed dwords and row scales are read two slices ahead (LA = 2), so the next step's row
-    // scales are made in slice 1 (JW) instead of slice 2. With two MFMAs a slice (MB = 2) the
-    // code-book reads follow stage A in the first gap and the scaling takes the second; the row
-    // scales take both gaps of slice 1.
+    // Stage positions: the MFMA index after which a part of a stage runs. Slice j reads the row scales
+    // (A) and code-book values (B, per packed byte e) of slice j + LA and packs the weights of slice
+    // j + 1 (products M, conversions C, per pair e), spread over the gaps as in the forward kernel.
+    // With few MFMAs a slice (MB = 2, 4) a slice is over before its LDS reads are back: they run two
+    // slices ahead, at MB = 2 the dY fragments too (LX), four dY buffers (step t + 3 loads into step
+    // t - 1's, whose readers are long done) leave the boundary (slice JB) nothing to drain, and the
+    // next step's row scales are made in slice 1 (JW) instead of slice 2.
     constexpr bool P2 = MB <= 4;
-    constexpr int LA = P2 ? 2 : 1, JW = P2 ? 1 : 2;
-    constexpr int qB = MB >= 7 ? 2 : (MB >= 4 ? 1 : 0), qC = MB >= 7 ? MB - 2 : MB - 1;
+    constexpr int LA = P2 ? 2 : 1, LX = MB <= 2 ? 2 : 1, JW = P2 ? 1 : 2, JB = 4 - LX;
+    constexpr int DBUFS = bwd8_dbufs(MB);
+    constexpr int B0 = MB > 7 ? 1 : 0, B1 = MB > 2 ? B0 + 1 : 0;  // B of bytes 0, 1 and 2, 3
+    auto at_M = [](int e) constexpr { return MB > 4 ? MB - 5 + e : (MB > 2 ? 1 + e / 2 : 1); };
+    auto at_C = [](int e) constexpr { return MB > 4 ? MB - 4 + e : (MB > 2 ? 2 + e / 2 : 1); };
     // next step's row scales
     constexpr int qS1 = MB >= 4 ? 1 : 0, qS2 = MB >= 7 ? 3 : (MB >= 4 ? 2 : 1), qS3 = MB >= 7 ? 5 : (MB >= 4 ? 3 : 1);
-    static_assert(qS3 < MB && qB < qC, "stages inside the slice");
+    static_assert(qS3 < MB && JW < JB && JW + LA >= 3, "stages inside the slice, a step's last look-ups before its tr reads move on");
     static_assert(MB <= 4 || DPT + 1 < MB, "a step's load parts fit one slice's MFMA gaps");
 
     // SwiGLU mode: this thread's two 16-byte chunks (row ch / 32, columns 8 (ch % 32) ..) of
@@ -208,6 +214,7 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
         const int t0 = max(cs0, sb), t1 = min(cs1, sb + sgpr(G.nsteps));
         if (t0 >= t1) continue;
         const int N = sgpr((int)G.w.n);
+        const int t_tail = N % kBwdBC != 0 ? sb + sgpr(G.nsteps) - 1 : -1;  // the group's partial step
         const int lddy = sgpr(G.lddy);
         const _Float16* const gdy = sgpr(G.dy);
         const uint32_t dy_bytes = sgpr(G.dy_bytes);
@@ -265,42 +272,37 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
         // at M = 8192).
         auto load_part = [&](int p, int t, int rd, int rw, bool live) __attribute__((always_inline)) {
             const int n0 = (t - sb) * kBwdBC;
-            const bool tail = n0 + kBwdBC > N;  // uniform
             if (p < DPT) {
                 const rsrc_t drs = make_rsrc(gdy + n0, live ? dy_bytes - 2u * (uint32_t)n0 : 0u);
-                if (!tail) {
-                    bload128_lds(drs, dy_dst(rd, p), dyo[p]);
-                } else {
-                    // rows and dY columns past N read zeros. The empty volatile asm keeps this a
-                    // branch taken only on a group's last, partial step: merged with the plain
-                    // loads, the per-lane checks became selects on every step (~8% of the loop).
+                uint32_t off = dyo[p];
+                if (t == t_tail) {
+                    // dY columns past N read zeros. The empty volatile asm keeps this a branch taken
+                    // only on a group's last, partial step: as selects on every step the per-lane
+                    // checks took ~8% of the loop.
                     asm volatile("");
-                    bload128_lds(drs, dy_dst(rd, p), off_if(n0 + 8 * dy_col(p) < N, dyo[p]));
+                    off = off_if(n0 + 8 * dy_col(p) < N, off);
                 }
+                bload128_lds(drs, dy_dst(rd, p), off);
                 return;
             }
+            // weight rows past N lie past the end of the packed bytes (zeros), and scales_3 gives
+            // them the scale 0 whatever statistics they meet
             uint8_t* slot = wring + rw;
             if (p == DPT) {
                 const uint32_t pskip = (uint32_t)n0 * (uint32_t)(K >> 1);
                 const rsrc_t wrs = make_rsrc(gpk + pskip, live ? pk_bytes - pskip : 0u);
-                if (!tail) {
-                    bload128_lds(wrs, slot, po);
-                } else {
-                    asm volatile("");
-                    bload128_lds(wrs, slot, off_if(n0 + lane < N, po));
-                }
+                bload128_lds(wrs, slot, po);
                 return;
             }
             const uint32_t kb = ((uint32_t)n0 * (uint32_t)K) >> bs_shift;  // blocks before this step
-            const bool rok = !tail || n0 + lane < N;
             if constexpr (NESTED) {
                 const rsrc_t ars = make_rsrc(gam8 + kb, live ? am_bytes - kb : 0u);
                 const rsrc_t a2rs = make_rsrc(gam2, live ? am2_bytes : 0u);
-                bload8_lds(ars, slot + 1024, off_if(rok, so));
-                bload32_lds(a2rs, slot + 1280, off_if(rok && cok, ((blk0 + kb) >> bs2_shift) * 4u));
+                bload8_lds(ars, slot + 1024, so);
+                bload32_lds(a2rs, slot + 1280, off_if(cok, ((blk0 + kb) >> bs2_shift) * 4u));
             } else {
                 const rsrc_t ars = make_rsrc(gamf + kb, live ? am_bytes - 4u * kb : 0u);
-                bload32_lds(ars, slot + 1024, off_if(rok, so));
+                bload32_lds(ars, slot + 1024, so);
             }
         };
         // every load of step t (the prologue)
@@ -354,121 +356,110 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
         scales_2();
         scales_3(t0, 0);
 
-        half8_t xf[MB], w, wn;
-        u32x2_t tr[2];   // the step's transposed reads: this lane's nibbles of slices 0, 1 and 2, 3
-        uint32_t d0;     // next slice: this lane's nibbles of its 8 rows (row e at bits 4 e)
-        float4_t s0, s1; // ... their row scales
-        float v[8];      // ... their code-book values
-        uint32_t e0;     // two-slice pipeline: the nibbles and scales of the slice after
-        float4_t t0s, t1s;
+        half8_t xf[LX][MB], w;
+        u32x2_t tr[2];        // the step's transposed reads: this lane's nibbles of slices 0, 1 and 2, 3
+        uint32_t d[LA];       // a slice's 8 rows of this lane's column (row e at bits 4 e; slice j: j % LA)
+        float4_t sc[LA][2];   // ... their row scales
+        float v[LA][8];       // ... their code-book values
+        float pr[8];          // the next slice's products
+        u32x4_t wn;           // the next slice's weights
         auto fetch_tr = [&](int rw) __attribute__((always_inline)) { lds_tr4x2(wring + rw + pkl, tr[0], tr[1]); };
         auto stage_A = [&](int sidx, int j) __attribute__((always_inline)) {
-            const uint32_t dj = tr[j >> 1][j & 1];
-            const float* sc = stab + 64 * sidx + 32 * g + 8 * j;
-            if constexpr (P2) {
-                e0 = dj;
-                t0s = *(const float4_t*)sc;
-                t1s = *(const float4_t*)(sc + 4);
-            } else {
-                d0 = dj;
-                s0 = *(const float4_t*)sc;
-                s1 = *(const float4_t*)(sc + 4);
-            }
+            d[j % LA] = tr[j >> 1][j & 1];
+            const float* s = stab + 64 * sidx + 32 * g + 8 * j;
+            sc[j % LA][0] = *(const float4_t*)s;
+            sc[j % LA][1] = *(const float4_t*)(s + 4);
         };
-        // two-slice pipeline: the slice after next becomes the next one
-        auto advance = [&]() __attribute__((always_inline)) {
-            if constexpr (P2) {
-                d0 = e0;
-                s0 = t0s;
-                s1 = t1s;
-            }
+        // byte e of d holds rows 2 e (low nibble) and 2 e + 1: one code-book pair each
+        auto stage_B = [&](int j, int e) __attribute__((always_inline)) {
+            const float2_t cv = *(const float2_t*)((const char*)lutT + byte_x8(d[j % LA], e));
+            v[j % LA][2 * e] = cv.x;
+            v[j % LA][2 * e + 1] = cv.y;
         };
-        auto stage_B = [&]() __attribute__((always_inline)) {
-            // byte b of d0 holds rows 2 b (low nibble) and 2 b + 1: one code-book pair each
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const float2_t cv = *(const float2_t*)((const char*)lutT + byte_x8(d0, b));
-                v[2 * b] = cv.x;
-                v[2 * b + 1] = cv.y;
-            }
+        auto stage_M = [&](int j, int e) __attribute__((always_inline)) {
+            pr[2 * e] = v[j % LA][2 * e] * sc[j % LA][e >> 1][2 * (e & 1)];
+            pr[2 * e + 1] = v[j % LA][2 * e + 1] * sc[j % LA][e >> 1][2 * (e & 1) + 1];
         };
-        auto stage_C = [&]() __attribute__((always_inline)) -> half8_t {
-            u32x4_t o;
-            o[0] = pack_half2(v[0] * s0[0], v[1] * s0[1]);
-            o[1] = pack_half2(v[2] * s0[2], v[3] * s0[3]);
-            o[2] = pack_half2(v[4] * s1[0], v[5] * s1[1]);
-            o[3] = pack_half2(v[6] * s1[2], v[7] * s1[3]);
-            return __builtin_bit_cast(half8_t, o);
-        };
+        auto stage_C = [&](int e) __attribute__((always_inline)) { wn[e] = pack_half2(pr[2 * e], pr[2 * e + 1]); };
         auto xfrag = [&](int rd, int i, int j) __attribute__((always_inline)) -> half8_t {
             return *(const half8_t*)(dring + rd + (32 * i + l32) * 128 + (((4 * g + j) ^ xsw) << 4));
         };
 
-        // slice 0 of the first step (and, two slices deep, slice 1's packed dwords and scales)
+        // the first slices of the first step
         fetch_tr(rw0);
-        stage_A(si0, 0);
-        advance();
 #pragma unroll
-        for (int i = 0; i < MB; ++i) xf[i] = xfrag(rd0, i, 0);
-        stage_B();
-        w = stage_C();
-        if constexpr (P2) {
-            stage_A(si0, 1);
-            advance();
+        for (int j = 0; j < LA; ++j) {
+            stage_A(si0, j);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) stage_B(j, e);
         }
+#pragma unroll
+        for (int j = 0; j < LX; ++j)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) xf[j][i] = xfrag(rd0, i, j);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            stage_M(0, e);
+            stage_C(e);
+        }
+        w = __builtin_bit_cast(half8_t, wn);
 
         for (int t = t0; t < t1; ++t) {
+            // step t + 3's dY buffer
+            const int rd3 = DBUFS == 3 ? rd0 : (rd0 == 0 ? 3 * DBUF : rd0 - DBUF);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int jn = (j + 1) & 3;
 #pragma unroll
                 for (int q = 0; q < MB; ++q) {
-                    acc[q] = mfma32x32x16(w, xf[q], acc[q]);
-                    if (j == 3 && q == 0) {
-                        // every wave's loads of step t+1 have landed (each waited in slice 1 or 2)
-                        // and every wave is past step t's slots: refill them with step t+3
-                        // (zeros past the segment's end), one part after each of this slice's
-                        // MFMAs. Past the last step the reads below see stale slots and their
-                        // values go unused.
-                        lds_barrier();
+                    acc[q] = mfma32x32x16(w, xf[j % LX][q], acc[q]);
+                    if (j == JB && q == 0) {
+                        // every wave's loads of step t+1 have landed (each waited in slice JW) and
+                        // every wave is past the slots that step t+3 (zeros past the segment's end)
+                        // loads into, one part after each of this slice's MFMAs. Past the last step
+                        // the reads below see stale slots and their values go unused.
+                        if constexpr (DBUFS == 4) bare_barrier();
+                        else lds_barrier();
                     }
                     if constexpr (MB > 4) {
-                        if (j == 3 && q <= DPT + 1) load_part(q, t + 3, rd0, rw0, t + 3 < t1);
-                    } else if (j == 3 && q == 0) {
+                        if (j == JB && q <= DPT + 1) load_part(q, t + 3, rd3, rw0, t + 3 < t1);
+                    } else if (j == JB && q == 0) {
                         // four MFMAs a slice leave no room to spread them (measured: the burst is
                         // 1.3% faster for the down-projection input gradient at MB = 4)
-                        load_step(t + 3, rd0, rw0, t + 3 < t1);
+                        load_step(t + 3, rd3, rw0, t + 3 < t1);
                     }
-                    // refill the dY fragment the MFMA above has read (slice j + 1)
-                    xf[q] = xfrag(j < 3 ? rd0 : rd1, q, jn);
-                    if (q == 0) {
-                        // step t+1's loads (this wave's) landed; its row scales follow in this
-                        // slice, before any stage A reads them
-                        const int ja = j + LA;  // the slice stage A prepares
-                        if (ja < 4) stage_A(si0, ja);
-                        else stage_A(1 - si0, ja - 4);
-                        if (j == JW) {
-                            // (slice 3's nibbles are out: the transposed reads move on a step)
+                    // refill the dY fragment the MFMA above has read (slice j + LX)
+                    xf[j % LX][q] = xfrag(j + LX < 4 ? rd0 : rd1, q, (j + LX) & 3);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (q == at_C(e) && at_C(e) > at_M(e)) stage_C(e);
+                        if (q == at_M(e)) stage_M(j + 1, e);
+                        if (q == at_C(e) && at_C(e) == at_M(e)) stage_C(e);
+                    }
+                    // slice j + LA's row scales and code-book values (of the next step past slice 3)
+                    if (q == 0) stage_A(j + LA < 4 ? si0 : 1 - si0, (j + LA) & 3);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (q == (e < 2 ? B0 : B1)) stage_B(j + LA, e);
+                    if (j == JW) {
+                        if (q == 0) {
+                            // step t+1's loads (this wave's) landed; its row scales follow in this
+                            // slice, before any stage A reads them (slice 3's nibbles are out: the
+                            // transposed reads move on a step)
                             wait_vmcnt<NL>();
                             fetch_tr(rw1);
                         }
-                    }
-                    if (j == JW) {
                         if (q == qS1) scales_1(rw1);
                         if (q == qS2) scales_2();
                         if (q == qS3) scales_3(t + 1, 1 - si0);
                     }
-                    if (q == qB) stage_B();
-                    if (q == qC) wn = stage_C();
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                w = wn;
-                advance();
+                w = __builtin_bit_cast(half8_t, wn);
             }
             // rotate the rings: step t + 1's buffers become the current ones
             rd0 = rd1;
             rw0 = rw1;
-            rd1 = rd1 == 2 * DBUF ? 0 : rd1 + DBUF;
+            rd1 = rd1 == (DBUFS - 1) * DBUF ? 0 : rd1 + DBUF;
             rw1 = rw1 == 2 * kB8WSlot ? 0 : rw1 + kB8WSlot;
             si0 = 1 - si0;
         }

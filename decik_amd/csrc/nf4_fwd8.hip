@@ -139,16 +139,9 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     }
     const float* const c2w = c2 + (glu ? 256 * (wave >> 2) : 0);  // this wave's weight's table
     const float offset = NESTED ? *W.offset : 0.0f;
+
     // byte offset of this wave's byte-pair code book in lut2
     const uint32_t book8 = (uint32_t)(glu ? 2048 * (wave >> 2) : 0);
-    // LDS byte address of the code-book pair of byte e of a packed dword
-    auto pair_addr = [&](uint32_t w, int e) __attribute__((always_inline)) -> uint32_t {
-        return (((w >> (8 * e)) & 0xFFu) << 3) + book8;
-    };
-    auto pair_at = [&](uint32_t addr) __attribute__((always_inline)) -> float2_t {
-        return *(const float2_t*)((const char*)lut2 + addr);
-    };
-
     const int wrow = nw0 + arow_to_n(l32);  // this lane's A row
     const bool rowok = wrow < N;
     const int xsw = (l32 >> 1) & 7;          // LDS swizzle of this lane's X rows
@@ -296,27 +289,11 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
         p = *(const u32x4_t*)(ws + 16 * lane);
         scale_1(ws);
     };
-    half8_t xf[LX][MB], w, wn;
-    uint32_t pa[4];   // code-book pair addresses of a slice's 4 packed bytes
+    half8_t xf[LX][MB], w;
+    uint32_t pa[4];   // code-book offsets of a slice's 4 packed bytes
     float v[LB][8];   // code-book values (slice j: v[j % LB])
-    auto stage_A = [&](uint32_t d) __attribute__((always_inline)) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pa[e] = pair_addr(d, e);
-    };
-    auto stage_B = [&](float* vs) __attribute__((always_inline)) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float2_t cv = pair_at(pa[e]);
-            vs[2 * e] = cv.x;
-            vs[2 * e + 1] = cv.y;
-        }
-    };
-    auto stage_C = [&](const float* vs) __attribute__((always_inline)) -> half8_t {
-        u32x4_t o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = pack_half2(vs[2 * e] * s, vs[2 * e + 1] * s);
-        return __builtin_bit_cast(half8_t, o);
-    };
+    float pr[8];      // ... times the scale
+    u32x4_t wn;       // the next slice's weights
     fetch_step(rw0);
     scale_2();
     s = scale_3();
@@ -324,22 +301,44 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     for (int j = 0; j < LX; ++j)
 #pragma unroll
         for (int i = 0; i < MB; ++i) xf[j][i] = xfrag(xs + rx0, i, j);
+    auto stage_A = [&](uint32_t d, int e) __attribute__((always_inline)) { pa[e] = byte_x8(d, e) + book8; };
+    auto stage_B = [&](float* vs, int e) __attribute__((always_inline)) {
+        const float2_t cv = *(const float2_t*)((const char*)lut2 + pa[e]);
+        vs[2 * e] = cv.x;
+        vs[2 * e + 1] = cv.y;
+    };
+    auto stage_M = [&](const float* vs, int e) __attribute__((always_inline)) {
+        pr[2 * e] = vs[2 * e] * s;
+        pr[2 * e + 1] = vs[2 * e + 1] * s;
+    };
+    auto stage_C = [&](int e) __attribute__((always_inline)) { wn[e] = pack_half2(pr[2 * e], pr[2 * e + 1]); };
 #pragma unroll
-    for (int j = 0; j < LB; ++j) {
-        stage_A(p[j]);
-        stage_B(v[j]);
+    for (int j = 0; j < LB; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            stage_A(p[j], e);
+            stage_B(v[j], e);
+        }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        stage_M(v[0], e);
+        stage_C(e);
     }
-    w = stage_C(v[0]);
-    // Stage positions (MFMA index after which a stage runs). Slice j reads the code-book values of
-    // slice j + LB (addresses A, reads B) and packs the weights of slice j + 1 (C). With seven or
-    // more MFMAs a slice that is one slice ahead, the stages in gaps of their own. With fewer
+    w = __builtin_bit_cast(half8_t, wn);
+    // Stage positions: the MFMA index after which a part of a stage runs. Slice j looks up the values
+    // of slice j + LB (addresses A, reads B, per packed byte e) and packs the weights of slice j + 1
+    // (products M, conversions C, per pair e). With seven or more MFMAs a slice that is one slice
+    // ahead, the parts spread over the gaps: a gap that held a whole stage took longer than the
+    // two MFMAs (one of either wave) that it must hide behind, while others were empty. With fewer
     // (MB = 2, 4) a slice is over before its LDS reads are back, so code-book values are read two
     // slices ahead, at MB = 2 X fragments too, and four X buffers (step t + 3 loads into step
-    // t - 1's, whose readers are long done) leave the boundary nothing to drain. (One slice ahead
-    // and draining, a step took about 2100 cycles at MB = 2, twice the LDS's own time.)
+    // t - 1's, whose readers are long done) leave the boundary nothing to drain.
     // The next step's packed weights and statistics, a wave's own, are fetched in slice JF, their
     // scale follows by slice 3: neither is on the boundary's path.
-    constexpr int qA = 0, qB = MB > 4 ? 1 : 0, qC = MB > 4 ? MB - 3 : (MB > 2 ? 2 : 1);
+    constexpr int A1 = MB > 7 || MB == 4 ? 1 : 0;                        // A of bytes 2, 3 (0, 1: gap 0)
+    constexpr int B0 = MB > 7 ? 1 : 0, B1 = MB > 2 ? B0 + 1 : 0;         // B of bytes 0, 1 and 2, 3
+    auto at_M = [](int e) constexpr { return MB > 4 ? MB - 5 + e : (MB > 2 ? 1 + e / 2 : 1); };
+    auto at_C = [](int e) constexpr { return MB > 4 ? MB - 4 + e : (MB > 2 ? 2 + e / 2 : 1); };
     constexpr int jS2 = MB > 4 ? JF : JF + 1, qS2 = MB > 4 ? MB - 3 : 0, qS3 = MB > 4 ? 1 : 0;
     // loads that may be in flight when step t+1's packed weights and statistics are fetched
     constexpr int NF = spread_after_stats(NP, SL, LX, JF);
@@ -368,20 +367,27 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
                 }
                 // refill the X fragment the MFMA above has read (slice j + LX)
                 xf[j % LX][q] = xfrag(xs + (j + LX < 4 ? rx0 : rx1), q, (j + LX) & 3);
-                if (q == qA) {
-                    stage_A(p[(j + LB) & 3]);
-                    if (j == JF) {
-                        wait_vmcnt<NF>();
-                        fetch_step(rw1);
-                    }
-                }
-                if (q == qB) stage_B(v[(j + LB) % LB]);
                 if (j == jS2 && q == qS2) scale_2();
                 if (j == 3 && q == qS3) s = scale_3();
-                if (q == qC) wn = stage_C(v[(j + 1) % LB]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    // (conversions of the gap before's products first, unless both share a gap)
+                    if (q == at_C(e) && at_C(e) > at_M(e)) stage_C(e);
+                    if (q == at_M(e)) stage_M(v[(j + 1) % LB], e);
+                    if (q == at_C(e) && at_C(e) == at_M(e)) stage_C(e);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (q == (e < 2 ? 0 : A1)) stage_A(p[(j + LB) & 3], e);
+                    if (q == (e < 2 ? B0 : B1)) stage_B(v[(j + LB) % LB], e);
+                }
+                if (j == JF && q == A1) {
+                    wait_vmcnt<NF>();
+                    fetch_step(rw1);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            w = wn;
+            w = __builtin_bit_cast(half8_t, wn);
         }
         // rotate the rings: step t + 1's buffers become the current ones
         const int rxo = rx0, rwo = rw0;
