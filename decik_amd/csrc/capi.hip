@@ -181,9 +181,16 @@ constexpr double kSplitUs = 0.26;
 constexpr int64_t kSmallReduceOutputs = 300000;
 constexpr int kRowUnit = 32;              // token rows per row block
 
-// col_tiles: output column tiles of the launch for this variant's tile width.
+// SwiGLU epilogue of tiles of more than 128 tokens: each round of work-groups ends with its gate and
+// up tiles' reads, which smaller tiles overlap with their main loop. With 8 us a round the plans of
+// forced-plan sweeps come out right: 7B down at 512 / 1024 / 2048 / 4096 tokens 128-token tiles 163 /
+// 262 / 458 / 932 us, 224-token 113 / 222 / 379 / 740, 256-token 116 / 229 / 377 / 706; 1.5B at 830 /
+// 1664 tokens 49 / 98, 58 / 112, 61 / 75.
+constexpr double kSwigluRoundUs = 8.0;
+
+// col_tiles: output column tiles of the launch for this variant's tile width. swiglu: see above.
 double plan_time(const VariantCost& v, int64_t m, int64_t col_tiles, int64_t ncols, int steps,
-                 int splits, bool split_chain) {
+                 int splits, bool split_chain, bool swiglu = false) {
     const int64_t rows = (int64_t)kRowUnit * v.rows_blocks;
     const int64_t tiles = ((m + rows - 1) / rows) * col_tiles;
     const int64_t slots = (int64_t)num_cus() * v.per_cu;
@@ -198,6 +205,7 @@ double plan_time(const VariantCost& v, int64_t m, int64_t col_tiles, int64_t nco
         // one work-group per CU at most: each runs faster than with a busy neighbour
         t += per * v.step_us * v.lone;
     }
+    if (swiglu && v.rows_blocks > 4) t += (double)(full + (rem > 0)) * kSwigluRoundUs;
     if (splits > 1) t += (double)splits * m * ncols * 4.0 * 1e-6 * kPartialUsPerMB + kReduceLaunchUs;
     if (splits > 1 && split_chain && m * ncols <= kSmallReduceOutputs) t += splits * kSplitUs;
     return t;
@@ -211,7 +219,7 @@ template <typename ColTiles>
 const VariantCost* choose_plan(const VariantCost* vs, int nv, int64_t m, int64_t ncols, int steps,
                                ColTiles col_tiles_of, int* splits, int max_splits = 32,
                                int64_t max_partial_bytes = INT64_MAX, int min_splits = 1,
-                               bool split_chain = false) {
+                               bool split_chain = false, bool swiglu = false) {
     double best = 1e300;
     const VariantCost* pick = &vs[0];
     *splits = 1;
@@ -222,7 +230,7 @@ const VariantCost* choose_plan(const VariantCost* vs, int nv, int64_t m, int64_t
             const int per = steps > 0 ? (steps + s - 1) / s : 0;
             if (steps > 0 && (steps + per - 1) / per != s) continue;  // s splits must all get work
             if (s > 1 && (double)s * m * ncols * 4.0 > (double)max_partial_bytes) continue;
-            const double t = plan_time(v, m, col_tiles_of(v), ncols, steps, s, split_chain);
+            const double t = plan_time(v, m, col_tiles_of(v), ncols, steps, s, split_chain, swiglu);
             if (t < best * 0.999) {
                 best = t;
                 pick = &v;
@@ -288,16 +296,12 @@ constexpr VariantCost kFwdVariants[] = {{1, 4, kFwdBN, 3, 2.35, 0.65},
                                        {8, 8, kFwdBN, 1, 2.25, 0.90},
                                        {9, 8, kFwdBN, 1, 2.45, 0.90}};
 constexpr int kNumFwdVariants = sizeof(kFwdVariants) / sizeof(kFwdVariants[0]);
-// nf4_bwd8_kernel: eight waves of 32 output columns (256-column tiles); its SwiGLU epilogue
-// exists for rows_blocks <= 4, which come first.
+// nf4_bwd8_kernel: eight waves of 32 output columns (256-column tiles)
 constexpr VariantCost kBwdVariants[] = {{2, 8, 256, 1, 1.00, 1.0},
                                        {4, 8, 256, 1, 1.75, 0.90},
                                        {7, 8, 256, 1, 2.10, 0.90},
                                        {8, 8, 256, 1, 2.25, 0.90}};
 constexpr int kNumBwdVariants = sizeof(kBwdVariants) / sizeof(kBwdVariants[0]);
-constexpr int kNumBwdSwigluVariants = 2;  // rows_blocks 2 and 4
-static_assert(kBwdVariants[kNumBwdSwigluVariants - 1].rows_blocks == 4 &&
-              kBwdVariants[kNumBwdSwigluVariants].rows_blocks > 4, "SwiGLU-capable variants first");
 
 // The eight-wave variants come last: nf4_fwd8_kernel advances its load descriptors by whole
 // steps, so it needs k % 64 == 0 and blocks that do not straddle rows (k % blocksize == 0).
@@ -348,7 +352,7 @@ GemmPlan plan_bwd_compute(int64_t m, int64_t k, const int64_t* ns, int ngroups, 
     GemmPlan p{};
     p.steps = 0;
     for (int g = 0; g < ngroups; ++g) p.steps += (int)((ns[g] + kBwdBC - 1) / kBwdBC);
-    const int nv = swiglu ? kNumBwdSwigluVariants : kNumBwdVariants;
+    const int nv = kNumBwdVariants;
     no_split = no_split || swiglu;
     const VariantCost* v = plan_override("DECIK_BWD_PLAN", kBwdVariants, nv, p.steps, &p.splits);
     if (v != nullptr && no_split) p.splits = 1;
@@ -356,7 +360,7 @@ GemmPlan plan_bwd_compute(int64_t m, int64_t k, const int64_t* ns, int ngroups, 
     if (v == nullptr)
         v = choose_plan(kBwdVariants, nv, m, k, p.steps,
                         [k](const VariantCost& c) { return (k + c.bn - 1) / c.bn; }, &p.splits,
-                        no_split ? 1 : 32, max_partial_bytes);
+                        no_split ? 1 : 32, max_partial_bytes, 1, false, swiglu);
     p.mt = v->rows_blocks;
     p.waves = v->waves;
     p.n_tiles = (int)((k + v->bn - 1) / v->bn);

@@ -34,8 +34,8 @@
 //
 // Epilogue: each token block's 32 x 256 tile goes through LDS (the rings, after a barrier) and
 // leaves as whole rows: split-K partial slabs (reduced by splitk_reduce_kernel), dX in fp32 or
-// fp16, or (SwiGLU mode, MB <= 4) dgate / dup from the tile rounded to fp16 and the matching gate
-// and up tiles, which every thread fetches for all its token blocks as the kernel starts.
+// fp16, or (SwiGLU mode) dgate / dup from the tile rounded to fp16 and the matching gate and up
+// tiles, which every thread fetches as the kernel starts (MB <= 4) or two token blocks ahead.
 #include "gemm_common.h"
 
 namespace dk {
@@ -156,28 +156,31 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
     static_assert(qS3 < MB && JW < JB && JW + LA >= 3, "stages inside the slice, a step's last look-ups before its tr reads move on");
     static_assert(MB <= 4 || DPT + 1 < MB, "a step's load parts fit one slice's MFMA gaps");
 
-    // SwiGLU mode: this thread's two 16-byte chunks (row ch / 32, columns 8 (ch % 32) ..) of
-    // every token block's gate and up tiles, requested as the kernel starts so that their reads
-    // overlap the main loop (the tiles are read before any output is written: dgate / dup may
-    // alias gate / up). The main loop's waits count its own loads only; these are older, so they
-    // only make the first wait stricter.
-    constexpr int SWB = MB <= 4 ? MB : 1;
+    // SwiGLU mode: this thread's two 16-byte chunks (row ch / 32, columns 8 (ch % 32) ..) of a token
+    // block's gate and up tiles (read before any output is written: dgate / dup may alias gate / up).
+    // With few token blocks all are requested as the kernel starts, so that their reads overlap the
+    // main loop, whose waits count its own loads only (these are older and only make the first wait
+    // stricter). More would not fit the registers: with MB > 4 they are read in the epilogue, two
+    // blocks ahead, which costs less than the 128-token tiles' extra unpacking where launches are
+    // large (7B down at 2048 tokens: 458 -> 379 us, at 512 163 -> 113).
+    constexpr int SWB = MB <= 4 ? MB : 2;
     u32x4_t gv[SWB][2], uv[SWB][2];
-    if constexpr (MB <= 4) {
-        if (a.swiglu) {
+    auto fetch_gate_up = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < MB; ++i)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int ch = tid + kB8Threads * h, row = ch >> 5, cc = ch & 31;
-                    const int m = m0 + 32 * i + row, col = tile_k0 + 8 * cc;
-                    gv[i][h] = uv[i][h] = u32x4_t{0u, 0u, 0u, 0u};
-                    if (m < M && col < K) {
-                        gv[i][h] = *(const u32x4_t*)(a.gate + (int64_t)m * a.ldgu + col);
-                        uv[i][h] = *(const u32x4_t*)(a.up + (int64_t)m * a.ldgu + col);
-                    }
-                }
+        for (int h = 0; h < 2; ++h) {
+            const int ch = tid + kB8Threads * h, row = ch >> 5, cc = ch & 31;
+            const int m = m0 + 32 * i + row, col = tile_k0 + 8 * cc;
+            gv[i % SWB][h] = uv[i % SWB][h] = u32x4_t{0u, 0u, 0u, 0u};
+            if (m < M && col < K) {
+                gv[i % SWB][h] = *(const u32x4_t*)(a.gate + (int64_t)m * a.ldgu + col);
+                uv[i % SWB][h] = *(const u32x4_t*)(a.up + (int64_t)m * a.ldgu + col);
+            }
         }
+    };
+    if constexpr (MB <= 4) {
+        if (a.swiglu)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) fetch_gate_up(i);
     }
 
     // LoRA input-gradient terms GU_g . A_g first (split 0 only; trip count 0 without LoRA): A row
@@ -485,45 +488,47 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
         for (int a4 = 0; a4 < 4; ++a4)
             *(float4_t*)(lp + 32 * a4) = float4_t{v[4 * a4 + 1], v[4 * a4], v[4 * a4 + 3], v[4 * a4 + 2]};
     };
-    if constexpr (MB <= 4) {
-        if (a.swiglu) {
-            // dgate / dup from G = fp16(dY . W) and the gate / up chunks fetched at the start
-            constexpr int RB = kB8BN * 2 + 16;
+    if (a.swiglu) {
+        // dgate / dup from G = fp16(dY . W) and the gate / up chunks
+        if constexpr (MB > 4)
 #pragma unroll
-            for (int i = 0; i < MB; ++i) {
-                // G = fp16(dY . W) through LDS as 32 x 256 fp16 rows
-                uint8_t* buf = dring + (i & 1) * 32 * RB;
-                uint8_t* lp = buf + l32 * RB + colw * 2;
-                stage_half(lp, acc[i]);
-                lds_barrier();
+            for (int i = 0; i < SWB; ++i) fetch_gate_up(i);
+        constexpr int RB = kB8BN * 2 + 16;
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int ch = tid + kB8Threads * h, row = ch >> 5, cc = ch & 31;
-                    const u32x4_t Gv = *(const u32x4_t*)(buf + row * RB + cc * 16);
-                    const int m = m0 + 32 * i + row, col = tile_k0 + 8 * cc;
-                    u32x4_t dg, du;
+        for (int i = 0; i < MB; ++i) {
+            // G = fp16(dY . W) through LDS as 32 x 256 fp16 rows
+            uint8_t* buf = dring + (i & 1) * 32 * RB;
+            uint8_t* lp = buf + l32 * RB + colw * 2;
+            stage_half(lp, acc[i]);
+            lds_barrier();
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        // elements copied to scalars first: hipcc compiles __builtin_bit_cast of
-                        // a vector element (vec[q]) as element 0 whatever q is
-                        const uint32_t Gq = Gv[q], gq = gv[i][h][q], uq = uv[i][h][q];
-                        const half2_t G2 = __builtin_bit_cast(half2_t, Gq);
-                        const half2_t g2 = __builtin_bit_cast(half2_t, gq);
-                        const half2_t u2 = __builtin_bit_cast(half2_t, uq);
-                        float d0, d1, e0, e1;
-                        swiglu_bwd1((float)G2.x, (float)g2.x, (float)u2.x, d0, e0);
-                        swiglu_bwd1((float)G2.y, (float)g2.y, (float)u2.y, d1, e1);
-                        dg[q] = pack_half2(d0, d1);
-                        du[q] = pack_half2(e0, e1);
-                    }
-                    if (m < M && col < K) {
-                        *(u32x4_t*)(a.dgate + (int64_t)m * a.ldd + col) = dg;
-                        *(u32x4_t*)(a.dup + (int64_t)m * a.ldd + col) = du;
-                    }
+            for (int h = 0; h < 2; ++h) {
+                const int ch = tid + kB8Threads * h, row = ch >> 5, cc = ch & 31;
+                const u32x4_t Gv = *(const u32x4_t*)(buf + row * RB + cc * 16);
+                const int m = m0 + 32 * i + row, col = tile_k0 + 8 * cc;
+                u32x4_t dg, du;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    // elements copied to scalars first: hipcc compiles __builtin_bit_cast of
+                    // a vector element (vec[q]) as element 0 whatever q is
+                    const uint32_t Gq = Gv[q], gq = gv[i % SWB][h][q], uq = uv[i % SWB][h][q];
+                    const half2_t G2 = __builtin_bit_cast(half2_t, Gq);
+                    const half2_t g2 = __builtin_bit_cast(half2_t, gq);
+                    const half2_t u2 = __builtin_bit_cast(half2_t, uq);
+                    float d0, d1, e0, e1;
+                    swiglu_bwd1((float)G2.x, (float)g2.x, (float)u2.x, d0, e0);
+                    swiglu_bwd1((float)G2.y, (float)g2.y, (float)u2.y, d1, e1);
+                    dg[q] = pack_half2(d0, d1);
+                    du[q] = pack_half2(e0, e1);
+                }
+                if (m < M && col < K) {
+                    *(u32x4_t*)(a.dgate + (int64_t)m * a.ldd + col) = dg;
+                    *(u32x4_t*)(a.dup + (int64_t)m * a.ldd + col) = du;
                 }
             }
-            return;
+            if (MB > 4 && i + SWB < MB) fetch_gate_up(i + SWB);
         }
+        return;
     }
     // LoRA input-gradient terms of branches whose input went through dropout (split 0): per token
     // block, P = GU_g . A_g on its own, rounded to fp16 (the branch's fp16 input gradient), times
@@ -623,7 +628,7 @@ static hipError_t launch_bwd8_t(const BwdArgs& a, int grid, hipStream_t s) {
 }
 
 hipError_t launch_bwd8(const BwdArgs& a, int mb, int grid, hipStream_t s) {
-    if (a.swiglu && (mb > 4 || a.splits > 1)) return hipErrorInvalidValue;  // SwiGLU: MB <= 4, no split
+    if (a.swiglu && a.splits > 1) return hipErrorInvalidValue;  // the SwiGLU epilogue needs finished sums
 #define X(T) \
     if (mb == T) return a.nested ? launch_bwd8_t<T, true>(a, grid, s) : launch_bwd8_t<T, false>(a, grid, s);
     X(2) X(4) X(7) X(8)

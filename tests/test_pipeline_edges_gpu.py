@@ -1,0 +1,76 @@
+"""The fused GEMMs where their software pipelines begin and end: contractions of one to five 64-wide
+steps (the rings hold three or four), the input gradient's partial last step next to values that must
+not leak in, the SwiGLU epilogue on tiles of 224 and 256 tokens, and the small-M kernel's last items.
+Bounds: the parity bar of assert_close; fused against separate launches of one plan: the same bits."""
+
+import pytest
+import torch
+
+from helpers import assert_close, make_weight, randn16
+from oracle import nf4 as O
+
+pytestmark = pytest.mark.gpu
+
+ROWS = {2: 64, 4: 128, 7: 224, 8: 256, 9: 288}
+
+
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("blocks", [2, 4, 7, 8, 9])
+def test_forward_few_steps(blocks, steps, device, monkeypatch):
+    from decik_amd.nf4 import linear_forward
+
+    monkeypatch.setenv("DECIK_FWD_PLAN", f"{blocks},1,8")
+    m, n, k = ROWS[blocks] + 1, 264, 64 * steps
+    packed, qs, w = make_weight((n, k), seed=steps, device=device)
+    x = randn16((m, k), seed=10 + blocks, device=device)
+    (y,) = linear_forward(x, [dict(packed=packed, qs=qs)])
+    assert_close(y, O.linear_ref(x.cpu().numpy(), w), what=f"{blocks} blocks, {steps} steps")
+
+
+@pytest.mark.parametrize("n", [8, 56, 64, 72, 136, 200, 320])
+@pytest.mark.parametrize("blocks", [2, 4, 7, 8])
+def test_input_gradient_partial_step(blocks, n, device, monkeypatch):
+    """dY is a view of a wider tensor whose columns past N hold infinities and NaN."""
+    from decik_amd.nf4 import linear_backward
+
+    monkeypatch.setenv("DECIK_BWD_PLAN", f"{blocks},1")
+    m, k = ROWS[blocks] + 3, 288
+    packed, qs, w = make_weight((n, k), seed=n, device=device)
+    wide = torch.full((m, n + 72), float("inf"), dtype=torch.float16, device=device)
+    wide[:, n + 8:] = float("nan")
+    dy = wide[:, :n]
+    dy.copy_(randn16((m, n), seed=n + 1, device=device, std=1e-2))
+    dx = linear_backward([dict(packed=packed, qs=qs, dy=dy)], m, k)
+    assert_close(dx, O.linear_dx_ref(dy.contiguous().cpu().numpy(), w), what=f"{blocks} blocks, N={n}")
+
+
+@pytest.mark.parametrize("plan", ["7,1", "8,1"])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (224, 128, 256), (257, 72, 288), (449, 200, 544)])
+def test_bwd_swiglu_large_tiles(m, n, k, plan, device, monkeypatch):
+    from decik_amd.nf4 import linear_backward, linear_backward_swiglu
+    from decik_amd.swiglu import swiglu_bwd
+
+    monkeypatch.setenv("DECIK_BWD_PLAN", plan)
+    packed, qs, w = make_weight((n, k), seed=n + k, device=device)
+    dy = randn16((m, n), seed=m, device=device, std=1e-2)
+    gate, up = (randn16((m, k), seed=m + s, device=device) for s in (1, 2))
+    item = dict(packed=packed, qs=qs, dy=dy)
+    dg, du = linear_backward_swiglu(item, gate, up)
+    grad = linear_backward([item], m, k)
+    assert_close(grad, O.linear_dx_ref(dy.cpu().numpy(), w), what=f"{m}x{n}x{k}")
+    dg2, du2 = swiglu_bwd(grad, gate, up)
+    assert torch.equal(dg, dg2) and torch.equal(du, du2)
+    g, u = gate.clone(), up.clone()  # outputs over the inputs
+    dg3, du3 = linear_backward_swiglu(item, g, u, out=(g, u))
+    assert torch.equal(dg3, dg) and torch.equal(du3, du)
+
+
+@pytest.mark.parametrize("m", [9, 16, 17, 32])
+@pytest.mark.parametrize("k", [32, 128, 160, 1056])
+def test_small_m_last_items(m, k, device):
+    from decik_amd.nf4 import linear_forward
+
+    packed, qs, w = make_weight((2 ** 15 + 8, k), seed=k, device=device)
+    x = randn16((m, k), seed=m, device=device)
+    (y,) = linear_forward(x, [dict(packed=packed, qs=qs)])
+    assert_close(y, O.linear_ref(x.cpu().numpy(), w), what=f"m={m} k={k}")
