@@ -355,6 +355,9 @@ GemmPlan plan_bwd_compute(int64_t m, int64_t k, const int64_t* ns, int ngroups, 
     const int nv = kNumBwdVariants;
     no_split = no_split || swiglu;
     const VariantCost* v = plan_override("DECIK_BWD_PLAN", kBwdVariants, nv, p.steps, &p.splits);
+    // the SwiGLU epilogue never splits: on its larger tiles a forced plan with splits does not apply (on
+    // the smaller ones the splits alone are dropped)
+    if (v != nullptr && swiglu && v->rows_blocks > 4 && p.splits > 1) v = nullptr;
     if (v != nullptr && no_split) p.splits = 1;
     if (v != nullptr && p.splits > 1 && (double)p.splits * m * k * 4.0 > (double)max_partial_bytes) v = nullptr;
     if (v == nullptr)
