@@ -551,7 +551,7 @@ bool gemv_requested(int64_t m, int64_t k, const int64_t* ns, int ngroups) {
 // plan) the MFMA kernels.
 struct GluSmallM {
     enum Kernel { kMfma, kGemv, kSkinny } kernel = kMfma;
-    int row_tiles = 0;  // small-M kernel: row tiles per work-group, half of them gate's
+    int row_tiles = 0;  // small-M kernel: row tiles of each weight per work-group
 };
 GluSmallM glu_small_m(int64_t m, int64_t k, int64_t n, bool lora) {
     GluSmallM r;
@@ -570,28 +570,25 @@ GluSmallM glu_small_m(int64_t m, int64_t k, int64_t n, bool lora) {
         r.kernel = GluSmallM::kGemv;
         return r;
     }
-    // The small-M kernel's work-groups take 8 * row_tiles rows of both weights; a CU works off its
-    // share of them: the row tiles with the fewest rows on the busiest CU. Ties go to 4 tiles up to
-    // 16 token rows (two work-groups fit a CU, one's loads behind the other's sums: [13824, 5120]
-    // at 16 rows 39.3 us against 42.8 for 8 tiles and 47.2 for 2), then to the larger.
-    // Graph-replayed at 16 rows, us for 2 / 4 / 6 / 8 / 10 tiles: 7B 39.9 / 37.0 / 39.8 / 47.1 /
-    // 32.7 (80 rows at 2 and 10), 1.5B 14.3 / 14.6 / 13.2 / 15.5 / 18.4 (48 at 2 and 6).
+    // The small-M GLU kernel's work-groups take 16 * row_tiles rows of both weights; a CU works off
+    // its share of them: the row tiles with the fewest rows on the busiest CU, of those the most (one
+    // work-group with its loads for all of them). Graph-replayed, us for 1 .. 5 tiles: 7B at 16 rows
+    // 48.0 / 36.9 / 33.2 / 39.2 / 26.2, at 32 84.4 / 61.2 / 48.4 / 53.6 / 33.9 (80 rows at 1 and 5);
+    // 1.5B at 16 rows 14.9 / 13.3 / 10.5 / 11.9 / 13.6 (48 at 1 and 3), [13824, 5120] 56.4 / 38.1 /
+    // 47.2 / 30.1 / 34.8 (64 at 1, 2 and 4), [4864, 896] 7.2 / 5.8 / 7.2 / 8.8 / 9.7 (32 at 1 and 2).
     const int64_t cus = num_cus();
     int64_t rows = INT64_MAX;
-    for (int rt : {2, 6, 8, 10, 4}) {
-        if (m > 16 && rt != 4 && rt != 6) continue;
-        const int64_t wgs = (n + 8 * rt - 1) / (8 * rt), per_cu = (wgs + cus - 1) / cus * 8 * rt;
-        const bool tie = m <= 16 || rt > r.row_tiles;
-        if (per_cu < rows || (per_cu == rows && tie)) {
+    for (int rt = 1; rt <= 5; ++rt) {
+        const int64_t wgs = (n + 16 * rt - 1) / (16 * rt), per_cu = (wgs + cus - 1) / cus * 16 * rt;
+        if (per_cu <= rows) {
             rows = per_cu;
             r.row_tiles = rt;
         }
     }
-    // MFMA tiles take 128 rows of both weights a CU in about the time the small-M kernel takes for
-    // 135 of them up to 16 token rows and 117 past (7B: 54.3 us for 128, 32.7 for 80, 44.4-48.9
-    // for 96).
+    // MFMA tiles take 128 rows of both weights a CU (7B: 48.3 us) in about the time this kernel takes
+    // for 145 of them up to 16 token rows (26.2 us for 80) and 114 past (33.9)
     const int64_t mfma_rows = ((n + 127) / 128 + cus - 1) / cus * 128;
-    if (rows * (m <= 16 ? 95 : 110) > mfma_rows * 100) return r;
+    if (rows * (m <= 16 ? 90 : 112) > mfma_rows * 100) return r;
     r.kernel = GluSmallM::kSkinny;
     return r;
 }
@@ -889,8 +886,7 @@ static int linear_fwd_impl(const std::string& name, const uint16_t* x, int64_t m
         const hipStream_t st = static_cast<hipStream_t>(stream);
         if (gs.kernel == GluSmallM::kGemv) return check_hip(launch_gemv_glu(a, st), "dk_nf4_glu_fwd GEMV launch");
         a.splits = 1;
-        a.ksteps = a.ksteps_per_split = (int)((k + kSkinnyStep - 1) / kSkinnyStep);
-        const int64_t grid = (ns[0] + 8 * gs.row_tiles - 1) / (8 * gs.row_tiles);
+        const int64_t grid = (ns[0] + 16 * gs.row_tiles - 1) / (16 * gs.row_tiles);
         if (grid > INT32_MAX / 2) return fail(name + ": problem too large");
         return check_hip(launch_skinny_glu(a, gs.row_tiles, (int)grid, st), "dk_nf4_glu_fwd small-M launch");
     }

@@ -175,13 +175,12 @@ int gemv_waves(int64_t m, int64_t k, int64_t nrows);
 // each group's first row group. splits > 1: fp32 partial slabs, then splitk_reduce_kernel.
 constexpr int kSkinnyMaxM = 32;
 hipError_t launch_skinny(const FwdArgs& a, int row_tiles, int grid, hipStream_t s);
-// the GLU form: grid work-groups of 8 * row_tiles rows of gate and of up (row_tiles 2, 4,
-// 6, 8 or 10; past 16 token rows 4 or 6), no split
+// Gate and up with SwiGLU (no LoRA terms): nf4_skinny_glu_kernel, grid work-groups of 16 * row_tiles
+// (1 to 5) rows of both weights, no split
 hipError_t launch_skinny_glu(const FwdArgs& a, int row_tiles, int grid, hipStream_t s);
 // 8-wave forward kernel (32 weight rows x 32*mb tokens per wave), mb = 8 or 9
 hipError_t launch_fwd8(const FwdArgs& a, int mb, int grid, hipStream_t s);
-// 8-wave input-gradient kernel (32 output columns x 32*mb tokens per wave), mb = 2, 4, 7 or 8;
-// the SwiGLU epilogue with mb <= 4
+// 8-wave input-gradient kernel (32 output columns x 32*mb tokens per wave), mb = 2, 4, 7 or 8
 hipError_t launch_bwd8(const BwdArgs& a, int mb, int grid, hipStream_t s);
 hipError_t launch_splitk_reduce(const ReduceArgs& a, hipStream_t s);
 

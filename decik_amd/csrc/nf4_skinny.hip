@@ -21,11 +21,6 @@
 //   k0 + 32 g + 8 t + e (a permutation of the step's 128 k that A and B share).
 // - Dequantization as in the other kernels: byte-pair code book in LDS (one 8-byte read per
 //   packed byte), fp32 multiply by the block scale, one fp16 rounding: the reference's bits.
-// - GLU (gate and up with SwiGLU): half of a work-group's row tiles are gate's, half the same rows
-//   of up, so the epilogue holds both sums of an output and writes h = fp16(silu(gate) up); no
-//   split. Before, these launches ran on 64-token MFMA tiles, mostly padding: 7B gate and up at
-//   3 / 16 / 32 rows 54.7 / 54.3 / 56.6 -> 30.4 / 32.7 / 48.9 us, 1.5B at 4 / 16 / 32 rows
-//   25.9 / 26.0 / 26.1 -> 11.9 / 13.2 / 15.4 (graph-replayed).
 #include "gemm_common.h"
 
 namespace dk {
@@ -39,15 +34,12 @@ __host__ __device__ constexpr size_t skinny_smem_bytes(int mt, int rt) {
     return (size_t)kSkWaves * 16 * mt * (16 * rt + 1) * 4;
 }
 
-template <int MT, bool NESTED, int RT, bool GLU>
+template <int MT, bool NESTED, int RT>
 __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a) {
-    constexpr int NW = GLU ? 2 : 1;   // weights of a work-group
-    constexpr int WT = RT / NW;       // row tiles per weight (GLU: WT of gate, then WT of up)
-    static_assert(RT % NW == 0, "the same rows of both weights");
-    constexpr int kSkRows = 16 * WT;  // rows of each weight per work-group
+    constexpr int kSkRows = 16 * RT;  // weight rows per work-group
     constexpr int kSkPad = 16 * RT + 1;
-    __shared__ float2_t lut2[NW * 256];  // byte-pair code books of this work-group's weights
-    __shared__ float c2[NW * 256];       // nested statistics: the code2 tables
+    __shared__ float2_t lut2[256];  // byte-pair code book of this work-group's weight
+    __shared__ float c2[256];       // nested statistics: the code2 table
     extern __shared__ __attribute__((aligned(16))) float red[];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -57,40 +49,30 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
     const int rg = (int)blockIdx.x / a.splits;  // row group over all groups' rows
     const int split = (int)blockIdx.x - rg * a.splits;
     int gi = 0;
-    if constexpr (!GLU) {
 #pragma unroll
-        for (int q = 1; q < kMaxGroups; ++q)
-            if (q < a.ngroups && rg >= a.g[q].tile_begin) gi = q;
-        gi = __builtin_amdgcn_readfirstlane(gi);
-    }
+    for (int q = 1; q < kMaxGroups; ++q)
+        if (q < a.ngroups && rg >= a.g[q].tile_begin) gi = q;
+    gi = __builtin_amdgcn_readfirstlane(gi);
     const FwdGroupDev& G = a.g[gi];
     const NF4Dev& W = G.w;
     const int M = a.m, K = a.k, N = (int)W.n, ldx = (int)a.ldx;
-    const int n0 = (GLU ? rg : rg - G.tile_begin) * kSkRows;
+    const int n0 = (rg - G.tile_begin) * kSkRows;
 
-    // the weights of the work-group (GLU: gate, up; one shape and block size)
-    rsrc_t wrs[NW], ars[NW], a2rs[NW];
-    float offset[NW], c2v[NW], book_hi[NW], book_lo[NW];
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        const NF4Dev& V = GLU ? a.g[w].w : W;
-        // (written to LDS once the first step's loads are on their way too)
-        book_hi[w] = V.code[(tid >> 4) & 15];
-        book_lo[w] = V.code[tid & 15];
-        if (NESTED && tid < 256) c2v[w] = V.code2[tid];
-        offset[w] = NESTED ? *V.offset : 0.0f;
-        wrs[w] = make_rsrc(V.packed, V.packed_bytes);
-        ars[w] = make_rsrc(NESTED ? (const void*)V.absmax8 : (const void*)V.absmaxf, V.absmax_bytes);
-        a2rs[w] = make_rsrc(V.absmax2, NESTED ? V.absmax2_bytes : 0u);
-    }
+    // (the tables are written to LDS once the first step's loads are on their way too)
+    const float book_hi = W.code[(tid >> 4) & 15], book_lo = W.code[tid & 15];
+    const float c2v = NESTED && tid < 256 ? W.code2[tid] : 0.0f;
+    const float offset = NESTED ? *W.offset : 0.0f;
+    const rsrc_t wrs = make_rsrc(W.packed, W.packed_bytes);
+    const rsrc_t ars = make_rsrc(NESTED ? (const void*)W.absmax8 : (const void*)W.absmaxf, W.absmax_bytes);
+    const rsrc_t a2rs = make_rsrc(W.absmax2, NESTED ? W.absmax2_bytes : 0u);
     const rsrc_t xrs = make_rsrc(a.x, a.x_bytes);
     const uint32_t bs_shift = W.bs_shift, bs2_shift = W.bs2_shift;
 
     // this lane's rows (A row i of tile r) and token rows (B column i of token block b)
-    uint32_t wbase[WT];
-    bool rok[WT];
+    uint32_t wbase[RT];
+    bool rok[RT];
 #pragma unroll
-    for (int r = 0; r < WT; ++r) {
+    for (int r = 0; r < RT; ++r) {
         const int row = n0 + 16 * r + i;
         rok[r] = row < N;
         wbase[r] = (uint32_t)(rok[r] ? row : 0) * (uint32_t)K + 32u * (uint32_t)g;  // flat element index
@@ -121,15 +103,14 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
         const bool kok = ss < s1 && k < K;  // K % 32 == 0: a lane's 32 k are wholly in or out
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-            const int w = r / WT, rr = r % WT;
-            const uint32_t el = wbase[rr] + (uint32_t)ss * kSkStep;
-            st.p[r] = bload128(wrs[w], off_if(kok && rok[rr], el >> 1));
+            const uint32_t el = wbase[r] + (uint32_t)ss * kSkStep;
+            st.p[r] = bload128(wrs, off_if(kok && rok[r], el >> 1));
             const uint32_t blk = el >> bs_shift;
             if constexpr (NESTED) {
-                st.q8[r] = bload8(ars[w], off_if(kok && rok[rr], blk));
-                st.s[r] = bloadf(a2rs[w], off_if(kok && rok[rr], (blk >> bs2_shift) * 4u));
+                st.q8[r] = bload8(ars, off_if(kok && rok[r], blk));
+                st.s[r] = bloadf(a2rs, off_if(kok && rok[r], (blk >> bs2_shift) * 4u));
             } else {
-                st.s[r] = bloadf(ars[w], off_if(kok && rok[rr], blk * 4u));
+                st.s[r] = bloadf(ars, off_if(kok && rok[r], blk * 4u));
             }
         }
 #pragma unroll
@@ -142,23 +123,21 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
     // are read while the one before is packed (the scheduling barriers keep that order: left to
     // itself the compiler waits for each item's four reads as soon as they are issued), and one wait
     // covers the four. Two waves a SIMD issue an instruction every 4 to 5 cycles between them, so it
-    // is the instructions per item that count, 34 before and 24 now. 7B at 16 rows: gate and up 28.3
-    // -> 25.3 us, q/k/v 8.7 -> 7.8; reading two items ahead was no faster, nor was a code book with
+    // is the instructions per item that count, 34 before and 24 now. 7B at 16 rows: gate and up in
+    // one launch 28.3 -> 25.3 us, q/k/v 8.7 -> 7.8; reading two items ahead was no faster, nor was a code book with
     // one copy per pair of LDS banks, which takes the bank conflicts out of every read (26.5 -> 28.2).
     auto compute = [&](Step& st) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-            const int w = r / WT;
-            if constexpr (NESTED) st.s[r] = c2[256 * w + st.q8[r]] * st.s[r] + offset[w];  // two roundings (no contraction)
-            if (!rok[r % WT]) st.s[r] = 0.0f;
+            if constexpr (NESTED) st.s[r] = c2[st.q8[r]] * st.s[r] + offset;  // two roundings (no contraction)
+            if (!rok[r]) st.s[r] = 0.0f;
         }
         float v[2][8];
         auto look = [&](int item) __attribute__((always_inline)) {
-            const int r = item / 4;
-            const uint32_t w = st.p[r][item % 4];
+            const uint32_t w = st.p[item / 4][item % 4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float2_t cv = *(const float2_t*)((const char*)lut2 + 2048 * (r / WT) + byte_x8(w, e));
+                const float2_t cv = *(const float2_t*)((const char*)lut2 + byte_x8(w, e));
                 v[item % 2][2 * e] = cv.x;
                 v[item % 2][2 * e + 1] = cv.y;
             }
@@ -187,10 +166,9 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
     Step sa, sb;
     int ss = s0 + wave;
     load(ss, sa);
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        if (tid < 256) lut2[256 * w + tid] = float2_t{book_hi[w], book_lo[w]};
-        if (NESTED && tid < 256) c2[256 * w + tid] = c2v[w];
+    if (tid < 256) {
+        lut2[tid] = float2_t{book_hi, book_lo};
+        if (NESTED) c2[tid] = c2v;
     }
     __syncthreads();  // the code book in LDS (the first step's loads are already in flight)
     while (ss < s1) {
@@ -221,36 +199,24 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
         const int m = t / kSkRows, row = t - m * kSkRows;  // consecutive threads: consecutive rows
         const int n = n0 + row;
         if (m >= M || n >= N) continue;
-        float v[NW];
+        float v = 0.0f;
 #pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            v[i] = 0.0f;
-#pragma unroll
-            for (int w = 0; w < kSkWaves; ++w) v[i] += red[(w * 16 * MT + m) * kSkPad + i * kSkRows + row];
-        }
-        if constexpr (GLU) {
-            // gate and up rounded to fp16 (their outputs), then the SwiGLU kernel's arithmetic
-            const float bg = a.g[0].bias != nullptr ? (float)a.g[0].bias[n] : 0.0f;
-            const float bu = a.g[1].bias != nullptr ? (float)a.g[1].bias[n] : 0.0f;
-            const uint32_t g2 = pack_half2(v[0] + bg, 0.0f), u2 = pack_half2(v[1] + bu, 0.0f);
-            if (a.g[0].y != nullptr) *(uint16_t*)(a.g[0].y + (int64_t)m * a.g[0].ldy + n) = (uint16_t)g2;
-            if (a.g[1].y != nullptr) *(uint16_t*)(a.g[1].y + (int64_t)m * a.g[1].ldy + n) = (uint16_t)u2;
-            *(uint16_t*)(a.h + (int64_t)m * a.ldh + n) = (uint16_t)swiglu_fwd2(g2, u2);
-        } else if (split_out) {
-            a.partials[((int64_t)split * M + m) * a.ncols + G.col_begin + n] = v[0];
+        for (int w = 0; w < kSkWaves; ++w) v += red[(w * 16 * MT + m) * kSkPad + row];
+        if (split_out) {
+            a.partials[((int64_t)split * M + m) * a.ncols + G.col_begin + n] = v;
         } else {
-            if (G.bias != nullptr) v[0] += (float)G.bias[n];
-            G.y[(int64_t)m * G.ldy + n] = to_half(v[0]);
+            if (G.bias != nullptr) v += (float)G.bias[n];
+            G.y[(int64_t)m * G.ldy + n] = to_half(v);
         }
     }
 }
 
-template <int MT, bool NESTED, int RT, bool GLU = false>
+template <int MT, bool NESTED, int RT>
 static hipError_t launch_skinny_t(const FwdArgs& a, int grid, hipStream_t s) {
     const size_t lds = skinny_smem_bytes(MT, RT);
-    const hipError_t e = allow_dynamic_lds((const void*)nf4_skinny_kernel<MT, NESTED, RT, GLU>, lds);
+    const hipError_t e = allow_dynamic_lds((const void*)nf4_skinny_kernel<MT, NESTED, RT>, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((nf4_skinny_kernel<MT, NESTED, RT, GLU>), dim3(grid), dim3(kSkThreads), lds, s, a);
+    hipLaunchKernelGGL((nf4_skinny_kernel<MT, NESTED, RT>), dim3(grid), dim3(kSkThreads), lds, s, a);
     return hipGetLastError();
 }
 
@@ -268,31 +234,6 @@ hipError_t launch_skinny(const FwdArgs& a, int row_tiles, int grid, hipStream_t 
         case 4: return launch_skinny_rt<4>(a, grid, s);
         case 5: return launch_skinny_rt<5>(a, grid, s);
         case 6: return launch_skinny_rt<6>(a, grid, s);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-template <int MT, int RT>
-static hipError_t launch_skinny_glu_t(const FwdArgs& a, int grid, hipStream_t s) {
-    return a.nested ? launch_skinny_t<MT, true, RT, true>(a, grid, s) : launch_skinny_t<MT, false, RT, true>(a, grid, s);
-}
-
-// GLU: grid work-groups of 8 * row_tiles rows of both weights (row_tiles even), no split
-hipError_t launch_skinny_glu(const FwdArgs& a, int row_tiles, int grid, hipStream_t s) {
-    if (a.m < 1 || a.m > kSkinnyMaxM || !a.glu || a.ngroups != 2 || a.g[0].w.n != a.g[1].w.n || a.h == nullptr ||
-        a.splits != 1 || a.g[0].lora_u != nullptr || a.g[1].lora_u != nullptr)
-        return hipErrorInvalidValue;
-    // two token blocks: 4 or 6 tiles (8 spilled registers, 2 were slower than 4 on every shape)
-    if (a.m > 16) {
-        if (row_tiles == 4) return launch_skinny_glu_t<2, 4>(a, grid, s);
-        return row_tiles == 6 ? launch_skinny_glu_t<2, 6>(a, grid, s) : hipErrorInvalidValue;
-    }
-    switch (row_tiles) {
-        case 2: return launch_skinny_glu_t<1, 2>(a, grid, s);
-        case 4: return launch_skinny_glu_t<1, 4>(a, grid, s);
-        case 6: return launch_skinny_glu_t<1, 6>(a, grid, s);
-        case 8: return launch_skinny_glu_t<1, 8>(a, grid, s);
-        case 10: return launch_skinny_glu_t<1, 10>(a, grid, s);
         default: return hipErrorInvalidValue;
     }
 }

@@ -74,3 +74,25 @@ def test_small_m_last_items(m, k, device):
     x = randn16((m, k), seed=m, device=device)
     (y,) = linear_forward(x, [dict(packed=packed, qs=qs)])
     assert_close(y, O.linear_ref(x.cpu().numpy(), w), what=f"m={m} k={k}")
+
+
+@pytest.mark.parametrize("nested", [True, False])
+@pytest.mark.parametrize("m,n,k", [
+    (3, 16, 64), (16, 4872, 512), (17, 1000, 576), (32, 8968, 640),  # 1, 2, 1, 3 row tiles; 1 to 5 super-steps
+    (9, 13832, 1088), (32, 18952, 1152),                            # 4, 5 row tiles; 9 super-steps
+])
+def test_small_m_glu_edges(m, n, k, nested, device):
+    from decik_amd.nf4 import glu_forward, launch_plan
+    from decik_amd.swiglu import swiglu_fwd
+
+    assert launch_plan(False, m, k, [n, n], glu=True, nested=nested)["kernel"] == "nf4_skinny_kernel"
+    items, ws = [], []
+    for s in range(2):
+        p, q, w = make_weight((n, k), seed=n + s, device=device, nested=nested)
+        items.append(dict(packed=p, qs=q))
+        ws.append(w)
+    x = randn16((m, k), seed=m, device=device)
+    g, u, h = glu_forward(x, *items)
+    for out, w in zip((g, u), ws):
+        assert_close(out, O.linear_ref(x.cpu().numpy(), w), what=f"{m}x{n}x{k}")
+    assert torch.equal(h, swiglu_fwd(g, u))
