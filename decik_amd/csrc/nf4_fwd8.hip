@@ -60,7 +60,7 @@ __host__ __device__ constexpr size_t fwd8_smem_bytes(int mb) {
     return kF8Header + kF8Dummy + (size_t)fwd8_xring_bytes(mb) + kF8Waves * 3 * (size_t)kF8WSlot;
 }
 
-template <int MB, bool NESTED>
+template <int MB, bool NESTED, bool GLU>
 __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a) {
     constexpr int BM = 32 * MB;
     constexpr int XBUF = BM * 128;                               // bytes of one X ring buffer
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS bases stay scalar
     const int l32 = lane & 31, g = lane >> 5;
     const bool wide = a.wide_stats != 0;
-    const bool glu = a.glu != 0;
+    constexpr bool glu = GLU;
     const int wslot_bytes = kF8WSlot;
 
     const int L = xcd_logical_id();
@@ -140,8 +140,9 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     const float* const c2w = c2 + (glu ? 256 * (wave >> 2) : 0);  // this wave's weight's table
     const float offset = NESTED ? *W.offset : 0.0f;
 
-    // byte offset of this wave's byte-pair code book in lut2
-    const uint32_t book8 = (uint32_t)(glu ? 2048 * (wave >> 2) : 0);
+    // byte offset of this wave's byte-pair code book in lut2 (GLU: a 64-token step is bound by the
+    // instructions it issues, so the launches of one weight do not carry the addition)
+    const uint32_t book8 = 2048u * (uint32_t)(wave >> 2);
     const int wrow = nw0 + arow_to_n(l32);  // this lane's A row
     const bool rowok = wrow < N;
     const int xsw = (l32 >> 1) & 7;          // LDS swizzle of this lane's X rows
@@ -301,7 +302,7 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     for (int j = 0; j < LX; ++j)
 #pragma unroll
         for (int i = 0; i < MB; ++i) xf[j][i] = xfrag(xs + rx0, i, j);
-    auto stage_A = [&](uint32_t d, int e) __attribute__((always_inline)) { pa[e] = byte_x8(d, e) + book8; };
+    auto stage_A = [&](uint32_t d, int e) __attribute__((always_inline)) { pa[e] = byte_x8(d, e) + (GLU ? book8 : 0u); };
     auto stage_B = [&](float* vs, int e) __attribute__((always_inline)) {
         const float2_t cv = *(const float2_t*)((const char*)lut2 + pa[e]);
         vs[2 * e] = cv.x;
@@ -335,10 +336,13 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     // t - 1's, whose readers are long done) leave the boundary nothing to drain.
     // The next step's packed weights and statistics, a wave's own, are fetched in slice JF, their
     // scale follows by slice 3: neither is on the boundary's path.
+    // (MB = 2: two waves a SIMD issue an instruction every 4 to 5 cycles between them, and a step's 183
+    // to 199 instructions are its time. One wait a packing and no code-book offset without GLU made it
+    // so from 206: a 7B layer's projections at 64 tokens 115.3 -> 112.2 us.)
     constexpr int A1 = MB > 7 || MB == 4 ? 1 : 0;                        // A of bytes 2, 3 (0, 1: gap 0)
     constexpr int B0 = MB > 7 ? 1 : 0, B1 = MB > 2 ? B0 + 1 : 0;         // B of bytes 0, 1 and 2, 3
-    auto at_M = [](int e) constexpr { return MB > 4 ? MB - 5 + e : (MB > 2 ? 1 + e / 2 : 1); };
-    auto at_C = [](int e) constexpr { return MB > 4 ? MB - 4 + e : (MB > 2 ? 2 + e / 2 : 1); };
+    auto at_M = [](int e) constexpr { return MB > 4 ? MB - 5 + e : 1 + e / 2; };
+    auto at_C = [](int e) constexpr { return MB > 4 ? MB - 4 + e : 2 + e / 2; };
     constexpr int jS2 = MB > 4 ? JF : JF + 1, qS2 = MB > 4 ? MB - 3 : 0, qS3 = MB > 4 ? 1 : 0;
     // loads that may be in flight when step t+1's packed weights and statistics are fetched
     constexpr int NF = spread_after_stats(NP, SL, LX, JF);
@@ -369,12 +373,18 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
                 xf[j % LX][q] = xfrag(xs + (j + LX < 4 ? rx0 : rx1), q, (j + LX) & 3);
                 if (j == jS2 && q == qS2) scale_2();
                 if (j == 3 && q == qS3) s = scale_3();
+                if (MB == 2 && q == 1) {
+                    // a whole slice's packing in one gap: one wait for its code-book values (seven or
+                    // more LDS reads are younger), products before conversions
+                    __builtin_amdgcn_sched_barrier(0);
+                    wait_lgkmcnt<7>();
+                    __builtin_amdgcn_sched_barrier(0);
+                    wn = pack_half8(v[(j + 1) % LB], s);
+                }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    // (conversions of the gap before's products first, unless both share a gap)
-                    if (q == at_C(e) && at_C(e) > at_M(e)) stage_C(e);
+                for (int e = 0; e < 4 && MB > 2; ++e) {
+                    if (q == at_C(e)) stage_C(e);  // the gap before's products
                     if (q == at_M(e)) stage_M(v[(j + 1) % LB], e);
-                    if (q == at_C(e) && at_C(e) == at_M(e)) stage_C(e);
                 }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -496,18 +506,23 @@ __global__ __launch_bounds__(kF8Threads, 1) void nf4_fwd8_kernel(const FwdArgs a
     }
 }
 
-template <int MB, bool NESTED>
+template <int MB, bool NESTED, bool GLU>
 static hipError_t launch_fwd8_t(const FwdArgs& a, int grid, hipStream_t s) {
-    const hipError_t e = allow_dynamic_lds((const void*)nf4_fwd8_kernel<MB, NESTED>, fwd8_smem_bytes(MB));
+    const hipError_t e = allow_dynamic_lds((const void*)nf4_fwd8_kernel<MB, NESTED, GLU>, fwd8_smem_bytes(MB));
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((nf4_fwd8_kernel<MB, NESTED>), dim3(grid), dim3(kF8Threads),
+    hipLaunchKernelGGL((nf4_fwd8_kernel<MB, NESTED, GLU>), dim3(grid), dim3(kF8Threads),
                        fwd8_smem_bytes(MB), s, a);
     return hipGetLastError();
 }
 
+template <int MB, bool NESTED>
+static hipError_t launch_fwd8_n(const FwdArgs& a, int grid, hipStream_t s) {
+    return a.glu ? launch_fwd8_t<MB, NESTED, true>(a, grid, s) : launch_fwd8_t<MB, NESTED, false>(a, grid, s);
+}
+
 hipError_t launch_fwd8(const FwdArgs& a, int mb, int grid, hipStream_t s) {
 #define X(T) \
-    if (mb == T) return a.nested ? launch_fwd8_t<T, true>(a, grid, s) : launch_fwd8_t<T, false>(a, grid, s);
+    if (mb == T) return a.nested ? launch_fwd8_n<T, true>(a, grid, s) : launch_fwd8_n<T, false>(a, grid, s);
     X(2) X(4) X(7) X(8) X(9)
 #undef X
     return hipErrorInvalidValue;
