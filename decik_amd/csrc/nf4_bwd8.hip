@@ -25,12 +25,12 @@
 // and j + 1, one nibble per row in row order. A byte of that dword holds two rows of the lane's
 // column, so one byte-pair code-book entry (one 8-byte LDS read, its address one SDWA shift)
 // gives both codes; each is scaled by its own row's scale. The dY tile (32*MB x 64 fp16) is
-// shared by the work-group through a ring three steps deep, as in nf4_bwd_kernel. Row scales of
-// step t + 1 are computed during slice 2 of step t, one row per lane, and read back through a
-// per-wave LDS table. The loop is software-pipelined one slice ahead, as in the forward kernels:
-// stage A (transposed read every other slice, row scales of the next slice) after the slice's
-// first MFMA, stage B (code-book addresses and reads) after the third, stage C (scaling and fp16
-// packing) after the last but one, and each dY fragment refilled right after its MFMA read it.
+// shared by the work-group through a ring three (MB = 2, 4: four) steps deep. Row scales of
+// step t + 1 are computed during slice 2 (1 with MB = 2, 4) of step t, one row per lane, and read
+// back through a per-wave LDS table. The loop is software-pipelined one slice ahead (LDS reads two
+// with MB = 2, 4), as in the forward kernels: row scales, code-book addresses and reads, scaling and
+// fp16 packing of the next slices spread over a slice's MFMA gaps, each dY fragment refilled right
+// after its MFMA read it.
 //
 // Epilogue: each token block's 32 x 256 tile goes through LDS (the rings, after a barrier) and
 // leaves as whole rows: split-K partial slabs (reduced by splitk_reduce_kernel), dX in fp32 or

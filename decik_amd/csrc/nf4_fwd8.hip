@@ -18,12 +18,12 @@
 // g = lane / 32) and the row's block statistics, through a per-wave LDS ring three steps deep;
 // the X tile through a shared ring three steps deep (buffer_load ... lds). Slice j (16 of k) =
 // one unpacked dword of 8 weights (A operand) x MB X fragments (B operands). The loop is
-// software-pipelined one slice ahead: between the MFMAs of slice j the wave refills each X
-// fragment register right after its MFMA has read it and unpacks slice j + 1 in three stages
-// (code-book addresses, code-book reads, scaling and fp16 packing). Slice 3 holds the step
-// boundary (own-slot fetch, wait, barrier); the refill of the freed ring slots starts there and
-// continues through slices 0-2 of the next step, at most two loads per slice (spread_part), so
-// that the eight waves' loads do not queue up in one slice.
+// software-pipelined one slice ahead (its LDS reads two with MB = 2, 4): between the MFMAs of slice j
+// the wave refills each X fragment register right after its MFMA has read it and unpacks slice j + 1
+// (code-book offsets, code-book reads, scaling and fp16 packing, spread over the gaps). Slice 3 (2
+// at MB = 2) holds the step boundary (wait, barrier); the refill of the freed ring slots starts
+// there and continues through the next step's slices before it, at most two loads per slice
+// (spread_part), so that the eight waves' loads do not queue up in one slice.
 //
 // Epilogue: each token block's 32 x 256 output tile goes through LDS (the X ring, after a
 // barrier) and leaves as whole 512-byte rows; GLU tiles pair the gate wave (0..3) and up wave
