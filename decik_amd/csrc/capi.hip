@@ -570,25 +570,30 @@ GluSmallM glu_small_m(int64_t m, int64_t k, int64_t n, bool lora) {
         r.kernel = GluSmallM::kGemv;
         return r;
     }
-    // The small-M GLU kernel's work-groups take 16 * row_tiles rows of both weights; a CU works off
-    // its share of them: the row tiles with the fewest rows on the busiest CU, of those the most (one
-    // work-group with its loads for all of them). Graph-replayed, us for 1 .. 5 tiles: 7B at 16 rows
-    // 48.0 / 36.9 / 33.2 / 39.2 / 26.2, at 32 84.4 / 61.2 / 48.4 / 53.6 / 33.9 (80 rows at 1 and 5);
-    // 1.5B at 16 rows 14.9 / 13.3 / 10.5 / 11.9 / 13.6 (48 at 1 and 3), [13824, 5120] 56.4 / 38.1 /
-    // 47.2 / 30.1 / 34.8 (64 at 1, 2 and 4), [4864, 896] 7.2 / 5.8 / 7.2 / 8.8 / 9.7 (32 at 1 and 2).
+    // The small-M GLU kernel's work-groups take 16 * row_tiles rows of both weights. Beside its row tiles'
+    // unpacking a work-group reads X once, which costs as much as 0.6 + 0.08 m row tiles, and a CU works
+    // off its share of the work-groups: the row tiles with the least such work on the busiest CU, of
+    // those the most. Graph-replayed, us for 1 .. 5 tiles: 7B at 16 rows 55.7 / 43.3 / 38.0 / 43.8 / 28.7,
+    // at 32 97.2 / 69.2 / 55.8 / 61.6 / 38.2; 1.5B at 16 rows 15.4 / 13.8 / 10.6 / 12.1 / 13.9, at 32 27.3 /
+    // 22.7 / 14.7 / 15.9 / 18.7; [28672, 4096] at 16 rows 93.4 / 70.1 / 68.6 / 56.3 / 65.6 (by rows on the
+    // busiest CU alone one tile, the slowest, would win: 112 rows in seven work-groups).
     const int64_t cus = num_cus();
-    int64_t rows = INT64_MAX;
+    int64_t work = INT64_MAX;
     for (int rt = 1; rt <= 5; ++rt) {
-        const int64_t wgs = (n + 16 * rt - 1) / (16 * rt), per_cu = (wgs + cus - 1) / cus * 16 * rt;
-        if (per_cu <= rows) {
-            rows = per_cu;
+        const int64_t wgs = (n + 16 * rt - 1) / (16 * rt), per_cu = (wgs + cus - 1) / cus * (100 * rt + 60 + 8 * m);
+        if (per_cu <= work) {
+            work = per_cu;
             r.row_tiles = rt;
         }
     }
-    // MFMA tiles take 128 rows of both weights a CU (7B: 48.3 us) in about the time this kernel takes
-    // for 145 of them up to 16 token rows (26.2 us for 80) and 114 past (33.9)
-    const int64_t mfma_rows = ((n + 127) / 128 + cus - 1) / cus * 128;
-    if (rows * (m <= 16 ? 90 : 112) > mfma_rows * 100) return r;
+    // MFMA tiles (64 tokens, 128 rows of both weights) take the time of 11 row tiles each: at 8 / 16 /
+    // 24 / 32 rows small-M kernel against MFMA tiles [28672, 4096] 48.3 / 56.3 / 68.8 / 77.3 against 54.2 /
+    // 57.3 / 59.1 / 59.1 us, [24576, 4096] 40.2 / 48.0 / 60.5 / 69.5 against 52.3-55.4, [20544, 2048] 22.5 /
+    // 25.8 / 33.2 / 37.6 against 28.7-29.2, [25600, 1536] 19.7 / 22.6 / 28.2 / 30.9 against 24.6-25.1; in one
+    // round of five tiles a CU (7B at 32 rows 38.2 against 48.1, [20480, 3584] 38.7 against 48.5) or in two
+    // ([40960, 1024] 27.5 against 32.5, [36864, 5120] 112 against 137) the small-M kernel stays ahead
+    const int64_t mfma_work = ((n + 127) / 128 + cus - 1) / cus * 1100;
+    if (work > mfma_work) return r;
     r.kernel = GluSmallM::kSkinny;
     return r;
 }

@@ -303,6 +303,25 @@ def test_launch_plans():
     assert b"bad arguments" in L.dk_last_error()
 
 
+@pytest.mark.parametrize("n,k,small,tiled", [
+    (28672, 4096, (1, 2, 8), (17, 24, 32)), (28672, 8192, (1, 2, 8), (17, 24, 32)),
+    (24576, 4096, (1, 2, 8, 16), (24, 32)), (20544, 2048, (1, 2, 8, 16), (24, 32)), (25600, 1536, (1, 2, 8), (24, 32)),
+    # one work-group a CU, and two rounds of them against two of MFMA tiles
+    (18944, 3584, (1, 2, 8, 16, 24, 32), ()), (20480, 3584, (1, 2, 8, 16, 24, 32), ()), (40960, 1024, (1, 2, 8, 16, 32), ()),
+    (8960, 1536, (1, 2, 8, 16, 24, 32), ()),
+])
+def test_glu_plans_of_wide_weights(n, k, small, tiled):
+    """Gate and up at 1-32 rows leave the few-row kernels where a second round of their work-groups
+    takes longer than the MFMA tiles: measured at both sides of every line here (at [28672, 4096] and
+    32 rows 161 us on one row tile a work-group, 77 on four, 59 on MFMA tiles)."""
+    from decik_amd.nf4 import launch_plan
+
+    for rows, tiles in ((small, False), (tiled, True)):
+        for m in rows:
+            kernel = launch_plan(False, m, k, [n, n], glu=True, nested=True)["kernel"]
+            assert (kernel == "nf4_fwd8_kernel") == tiles, (m, n, k, kernel)
+
+
 def test_no_bit_cast_of_vector_elements():
     """hipcc compiles __builtin_bit_cast(T, v[i]) of an ext_vector_type element as element 0
     whatever i is (found twice in this library); the kernels copy elements to scalars first.
