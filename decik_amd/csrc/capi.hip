@@ -558,15 +558,19 @@ GluSmallM glu_small_m(int64_t m, int64_t k, int64_t n, bool lora) {
     if (lora || m < 1 || m > kSkinnyMaxM) return r;
     const char* forced = std::getenv("DECIK_FWD_PLAN");
     if (forced != nullptr && *forced != 0) return r;
-    // One row: the GEMV on every shape measured. Two rows: its second dot product costs in
-    // proportion to the weight (as in gemv_requested). Graph-replayed at two rows, GEMV against
-    // small-M kernel, us: [4864, 896] 7.0 against 7.2, 1.5B 10.8 against 11.5, [11008, 2048] 13.4
-    // against 15.0; 7B 32.8 against 28.7, [13824, 5120] 34-36 against 32.0. From 3 rows the
-    // small-M kernel wins on every shape (1.5B 14.7 against 11.9).
+    // One row: the GEMV, whose gate and up have the bits of the grouped launch of that row. It is the
+    // faster one on long rows and about even on the others: graph-replayed, GEMV against small-M kernel,
+    // us: [1024, 4096] 4.9 against 7.9, [13824, 5120] 25.2 against 28.1, [11008, 2048] 10.9 against 11.5,
+    // 7B 24.4 against 23.9, 1.5B 8.5 against 8.6, [4864, 896] 5.4 against 4.8, [8192, 3072] 12.4 against 10.1.
+    // Two rows: its second dot product costs in proportion to the weight, so only small weights of long
+    // rows, where the small-M kernel's four waves a weight make a long chain: [2048, 2048] 5.5 against
+    // 5.7, [2048, 6144] 9.9 against 12.0, [1024, 16384] 13.4 against 26.2, [64, 4096] 5.9 against 7.8. The
+    // others: [2048, 1536] 5.5 against 4.5, [4864, 896] 6.3 against 4.8, 1.5B 10.0 against 8.6, [11008, 2048]
+    // 12.2 against 11.6, 7B 28.9 against 24.0, [3072, 4096] 10.9 against 9.1, [2048, 8960] 18.0 against 14.2.
     const char* v = std::getenv("DECIK_SMALL_M");
     const bool gemv_forced = v != nullptr && std::string(v) == "gemv";
     const bool skinny_forced = v != nullptr && std::string(v) == "skinny";
-    if (!skinny_forced && gemv_glu_fits(m, k) && (m == 1 || gemv_forced || n * k < (int64_t(1) << 25))) {
+    if (!skinny_forced && gemv_glu_fits(m, k) && (m == 1 || gemv_forced || (k >= 2048 && n <= (k <= 6144 ? 2048 : 1024)))) {
         r.kernel = GluSmallM::kGemv;
         return r;
     }

@@ -322,6 +322,21 @@ def test_glu_plans_of_wide_weights(n, k, small, tiled):
             assert (kernel == "nf4_fwd8_kernel") == tiles, (m, n, k, kernel)
 
 
+@pytest.mark.parametrize("n,k,gemv", [
+    (64, 1536, False), (2048, 1536, False), (4864, 896, False), (8960, 1536, False),
+    (64, 2048, True), (2048, 2048, True), (3072, 2048, False), (11008, 2048, False),
+    (2048, 6144, True), (3072, 6144, False), (9728, 6144, False), (1024, 8960, True), (2048, 8960, False),
+    (1024, 16384, True), (3072, 16384, False), (18944, 3584, False),
+])
+def test_glu_plans_of_two_rows(n, k, gemv):
+    """Gate and up at two token rows: the GEMV where it was measured the faster of the two few-row
+    kernels (small weights of long rows), at one row always."""
+    from decik_amd.nf4 import launch_plan
+
+    assert (launch_plan(False, 2, k, [n, n], glu=True, nested=True)["kernel"] == "nf4_gemv_kernel") == gemv
+    assert launch_plan(False, 1, k, [n, n], glu=True, nested=True)["kernel"] == "nf4_gemv_kernel"
+
+
 def test_no_bit_cast_of_vector_elements():
     """hipcc compiles __builtin_bit_cast(T, v[i]) of an ext_vector_type element as element 0
     whatever i is (found twice in this library); the kernels copy elements to scalars first.

@@ -16,7 +16,9 @@ CASES = [
     (1, 8, 64, 64, True, "nf4_gemv_kernel"),           # one work-group, one chunk pair a row
     (1, 1544, 3584, 64, True, "nf4_gemv_kernel"),      # several loads a thread, a ragged last group
     (1, 40, 20480, 128, False, "nf4_gemv_kernel"),     # long rows: several loads a row
-    (2, 264, 1536, 64, True, "nf4_gemv_kernel"),
+    (2, 264, 1536, 64, True, "nf4_skinny_kernel"),     # two rows of short contractions
+    (2, 264, 2048, 64, True, "nf4_gemv_kernel"),       # ... and of longer ones
+    (2, 2056, 2048, 64, True, "nf4_skinny_kernel"),    # one row group past the GEMV's
     (2, 72, 8960, 64, False, "nf4_gemv_kernel"),
     (3, 8, 64, 64, True, "nf4_skinny_kernel"),         # fewer rows than a tile, half a super-step
     (3, 4864, 896, 64, True, "nf4_skinny_kernel"),     # 4 tiles
