@@ -18,7 +18,7 @@ MAX_GROUPS = 4
 PLAN_GLU, PLAN_LORA, PLAN_NO_SPLIT, PLAN_NESTED, PLAN_PARTS = 1, 2, 4, 8, 16
 # dk_nf4_linear_plan's kernel ids (2, an earlier input-gradient kernel, is no longer returned)
 PLAN_KERNELS = ("nf4_fwd_kernel", "nf4_fwd8_kernel", "retired", "nf4_bwd8_kernel", "nf4_gemv_kernel",
-                "nf4_skinny_kernel")
+                "nf4_skinny_kernel", "nf4_skinny_glu_kernel")
 
 _lib = None
 _lock = threading.Lock()

@@ -730,7 +730,7 @@ int dk_nf4_linear_plan(int backward, int64_t m, int64_t k, const int64_t* ns, in
         p.mt = gs.kernel == GluSmallM::kSkinny ? (m <= 16 ? 1 : 2) : 0;
         p.waves = 8;
         p.splits = 1;
-        kernel = gs.kernel == GluSmallM::kGemv ? 4 : 5;
+        kernel = gs.kernel == GluSmallM::kGemv ? 4 : 6;  // nf4_gemv_kernel, nf4_skinny_glu_kernel
     } else {
         p = plan_fwd(m, k, ns, ngroups, glu, k % 64 == 0 && k % blocksize == 0, single, 1,
                      !(glu && (flags & DK_PLAN_NESTED) != 0));

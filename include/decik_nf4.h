@@ -323,10 +323,12 @@ int dk_swiglu_bwd(const uint16_t* grad, const uint16_t* gate, const uint16_t* up
  * with at most 2^24 weights, 5-8 with fewer than 2^23 weights
  * and 8 k <= 32768, without LoRA terms; GLU launches of one token row, two with k >= 2048
  * and at most 2048 weight rows, 1024 past k = 6144), 5
- * nf4_skinny_kernel (such launches of up to 32 token rows otherwise, but past 16 rows not for
- * weights of more 64-row groups than the device has CUs, GLU launches not where its row groups
- * would outlast the MFMA tiles; out[2] is then its contraction splits); DECIK_SMALL_M = gemv / skinny picks one
- * of the two where both may run). Host-only (no GPU call);
+ * nf4_skinny_kernel (forward launches of up to 32 token rows without LoRA terms otherwise, but past
+ * 16 rows not for weights of more 96-row groups than the device has CUs; out[2] is then its
+ * contraction splits), 6 nf4_skinny_glu_kernel (such GLU launches otherwise, but not where further
+ * rounds of its work-groups would outlast the MFMA tiles, as at [28672, 4096] from 12 token rows on
+ * or [20544, 2048] from 24)); DECIK_SMALL_M = gemv / skinny picks the GEMV or the other few-row kernel where
+ * both may run. Host-only (no GPU call);
  * honours DECIK_FWD_PLAN / DECIK_BWD_PLAN / DECIK_SMALL_M like the launches. Returns 0, or nonzero
  * with dk_last_error() on bad arguments. */
 #define DK_PLAN_GLU 1

@@ -319,7 +319,8 @@ def test_glu_plans_of_wide_weights(n, k, small, tiled):
     for rows, tiles in ((small, False), (tiled, True)):
         for m in rows:
             kernel = launch_plan(False, m, k, [n, n], glu=True, nested=True)["kernel"]
-            assert (kernel == "nf4_fwd8_kernel") == tiles, (m, n, k, kernel)
+            few = "nf4_gemv_kernel" if m == 1 else "nf4_skinny_glu_kernel"
+            assert kernel == ("nf4_fwd8_kernel" if tiles else few), (m, n, k)
 
 
 @pytest.mark.parametrize("n,k,gemv", [
@@ -333,7 +334,8 @@ def test_glu_plans_of_two_rows(n, k, gemv):
     kernels (small weights of long rows), at one row always."""
     from decik_amd.nf4 import launch_plan
 
-    assert (launch_plan(False, 2, k, [n, n], glu=True, nested=True)["kernel"] == "nf4_gemv_kernel") == gemv
+    assert launch_plan(False, 2, k, [n, n], glu=True, nested=True)["kernel"] == \
+        ("nf4_gemv_kernel" if gemv else "nf4_skinny_glu_kernel")
     assert launch_plan(False, 1, k, [n, n], glu=True, nested=True)["kernel"] == "nf4_gemv_kernel"
 
 

@@ -1,7 +1,7 @@
 """The fused gate+up+SwiGLU forward at 1-32 token rows (the GEMV's and the small-M kernel's GLU
-forms): gate and up against the oracle, h the SwiGLU kernel's bits on them, the outputs optional,
-at the sizes where the forms' tiles end and where the dispatch changes. Gate and up carry code
-books and code2 tables of their own."""
+forms, MFMA tiles beyond): gate and up against the oracle, h the SwiGLU kernel's bits on them, the
+outputs optional, at the sizes where the forms' tiles end and where the dispatch changes. Gate and
+up carry code books and code2 tables of their own."""
 
 import pytest
 import torch
@@ -12,21 +12,23 @@ from oracle import nf4 as O
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # (m, n, k, blocksize, nested, kernel)
-    (1, 8, 64, 64, True, "nf4_gemv_kernel"),           # one work-group, one chunk pair a row
-    (1, 1544, 3584, 64, True, "nf4_gemv_kernel"),      # several loads a thread, a ragged last group
-    (1, 40, 20480, 128, False, "nf4_gemv_kernel"),     # long rows: several loads a row
-    (2, 264, 1536, 64, True, "nf4_skinny_kernel"),     # two rows of short contractions
-    (2, 264, 2048, 64, True, "nf4_gemv_kernel"),       # ... and of longer ones
-    (2, 2056, 2048, 64, True, "nf4_skinny_kernel"),    # one row group past the GEMV's
+    # (m, n, k, blocksize, nested, kernel); row tiles: of each weight, a work-group
+    (1, 8, 64, 64, True, "nf4_gemv_kernel"),               # one work-group, one chunk pair a row
+    (1, 1544, 3584, 64, True, "nf4_gemv_kernel"),          # several loads a thread, a ragged last group
+    (1, 40, 20480, 128, False, "nf4_gemv_kernel"),         # long rows: several loads a row
+    (2, 264, 1536, 64, True, "nf4_skinny_glu_kernel"),     # two rows of short contractions
+    (2, 264, 2048, 64, True, "nf4_gemv_kernel"),           # ... and of longer ones
+    (2, 2056, 2048, 64, True, "nf4_skinny_glu_kernel"),    # more rows than the GEMV takes
     (2, 72, 8960, 64, False, "nf4_gemv_kernel"),
-    (3, 8, 64, 64, True, "nf4_skinny_kernel"),         # fewer rows than a tile, half a super-step
-    (3, 4864, 896, 64, True, "nf4_skinny_kernel"),     # 4 tiles
-    (16, 8968, 192, 64, True, "nf4_skinny_kernel"),    # 6 tiles, a ragged last group
-    (8, 12296, 128, 64, False, "nf4_skinny_kernel"),   # 8 rows into the next tile count
-    (5, 18952, 256, 128, True, "nf4_skinny_kernel"),   # 10 tiles
-    (17, 1032, 1536, 64, True, "nf4_skinny_kernel"),   # two token blocks
-    (32, 12296, 128, 64, False, "nf4_skinny_kernel"),  # two token blocks, 6 tiles
+    (3, 8, 64, 64, True, "nf4_skinny_glu_kernel"),         # fewer rows than a tile, half a super-step
+    (3, 4864, 896, 64, True, "nf4_skinny_glu_kernel"),     # 2 row tiles
+    (16, 8968, 192, 64, True, "nf4_skinny_glu_kernel"),    # 3 row tiles, a ragged last group
+    (8, 12296, 128, 64, False, "nf4_skinny_glu_kernel"),   # 4 row tiles: 8 rows more than 3 would take
+    (5, 18952, 256, 128, True, "nf4_skinny_glu_kernel"),   # 5 row tiles
+    (17, 1032, 1536, 64, True, "nf4_skinny_glu_kernel"),   # two token blocks
+    (32, 12296, 128, 64, False, "nf4_skinny_glu_kernel"),  # two token blocks, 4 row tiles
+    (11, 28680, 128, 64, True, "nf4_skinny_glu_kernel"),   # two rounds of work-groups
+    (12, 28680, 128, 64, True, "nf4_fwd8_kernel"),         # ... which from here on outlast the MFMA tiles
 ]
 
 

@@ -85,7 +85,7 @@ def test_small_m_glu_edges(m, n, k, nested, device):
     from decik_amd.nf4 import glu_forward, launch_plan
     from decik_amd.swiglu import swiglu_fwd
 
-    assert launch_plan(False, m, k, [n, n], glu=True, nested=nested)["kernel"] == "nf4_skinny_kernel"
+    assert launch_plan(False, m, k, [n, n], glu=True, nested=nested)["kernel"] == "nf4_skinny_glu_kernel"
     items, ws = [], []
     for s in range(2):
         p, q, w = make_weight((n, k), seed=n + s, device=device, nested=nested)
