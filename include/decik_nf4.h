@@ -159,12 +159,16 @@ int dk_nf4_linear_rope_fwd(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
 
 /* Gate and up projections and SwiGLU in one launch: groups[0] = gate, groups[1] = up (one shape
  * [n, k]; bias and LoRA as in dk_nf4_linear_fwd), h = fp16(silu(gate) * up) [m, n] (row stride
- * ldh) from the fp16-rounded gate and up -- the same bits as dk_nf4_linear_fwd followed by
- * dk_swiglu_fwd. One launch when gate and up have the same statistics kind (both plain or both
- * nested, as bitsandbytes stores them), blocksize >= 64 and k % 64 == 0; then groups[i].y may be
- * NULL (not stored). Other weights run as the grouped launch then the SwiGLU kernel and need both
- * y, with rows contiguous (ldy = ldh = n). Up to 32 token rows without LoRA terms run the GLU forms
- * of the GEMV and the small-M kernel. No workspace. */
+ * ldh) from the fp16-rounded gate and up: dk_swiglu_fwd's bits on the gate and up that the call
+ * forms (and stores where y is given). Their fp32 sums run in the launch's own order -- at one
+ * token row that of dk_nf4_linear_fwd, otherwise one of three by row count (GEMV, small-M kernel,
+ * MFMA tiles) -- so a few of them round to the other neighbouring fp16 value than in
+ * dk_nf4_linear_fwd, or in a call of another row count. One launch when gate and up have the same
+ * statistics kind (both plain or both nested, as bitsandbytes stores them), blocksize >= 64 and
+ * k % 64 == 0; then groups[i].y may be NULL (not stored). Other weights run as the grouped launch
+ * then the SwiGLU kernel and need both y, with rows contiguous (ldy = ldh = n). Up to 32 token rows
+ * without LoRA terms run the GLU forms of the GEMV and the small-M kernel, but from 12 rows on not
+ * for every weight of more than 20480 rows (dk_nf4_linear_plan). No workspace. */
 int dk_nf4_glu_fwd(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
                    const dk_linear_fwd_group* groups, int lora_rank, uint16_t* h, int64_t ldh,
                    void* stream);

@@ -59,6 +59,28 @@ def test_glu_few_rows(m, n, k, blocksize, nested, kernel, device):
         assert torch.equal(g, g2) and torch.equal(u, u2)
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 16, 17, 32])
+def test_glu_few_rows_precision(m, device, monkeypatch):
+    """The few-row forms' sums are no worse than the MFMA tiles': the gate and up values that are not
+    the correctly rounded 64-bit sums, counted for both on the same inputs. Bound: the tiles' count
+    and three standard deviations of such a (Poisson) count."""
+    from decik_amd.nf4 import glu_forward
+
+    n, k = 8960, 1536
+    items, exact = [], []
+    x = randn16((m, k), seed=m, device=device)
+    for i in range(2):
+        p, q, w = make_weight((n, k), seed=40 + i, device=device)
+        items.append(dict(packed=p, qs=q))
+        exact.append((x.double().cpu() @ torch.from_numpy(w).double().T).half())
+    def misrounded():
+        return sum(int((y.cpu() != e).sum()) for y, e in zip(glu_forward(x, *items)[:2], exact))
+    few = misrounded()
+    monkeypatch.setenv("DECIK_FWD_PLAN", "2,1,8")
+    tiles = misrounded()
+    assert tiles > 0 and few <= tiles + 3 * tiles ** 0.5, (few, tiles)
+
+
 @pytest.mark.parametrize("m,n", [(1, 64), (4, 200), (20, 200)])
 def test_glu_few_rows_strided(m, n, device):
     """X and every output as rows of wider buffers; what lies beside them is not touched."""
