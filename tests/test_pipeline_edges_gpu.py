@@ -6,7 +6,7 @@ Bounds: the parity bar of assert_close; fused against separate launches of one p
 import pytest
 import torch
 
-from helpers import assert_close, make_weight, randn16
+from helpers import assert_close, make_weight, oracle_state, randn16
 from oracle import nf4 as O
 
 pytestmark = pytest.mark.gpu
@@ -14,17 +14,49 @@ pytestmark = pytest.mark.gpu
 ROWS = {2: 64, 4: 128, 7: 224, 8: 256, 9: 288}
 
 
+@pytest.mark.parametrize("nested", [True, False])
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5])
 @pytest.mark.parametrize("blocks", [2, 4, 7, 8, 9])
-def test_forward_few_steps(blocks, steps, device, monkeypatch):
-    from decik_amd.nf4 import linear_forward
+def test_forward_few_steps(blocks, steps, nested, device, monkeypatch):
+    from decik_amd.nf4 import launch_plan, linear_forward
 
     monkeypatch.setenv("DECIK_FWD_PLAN", f"{blocks},1,8")
     m, n, k = ROWS[blocks] + 1, 264, 64 * steps
-    packed, qs, w = make_weight((n, k), seed=steps, device=device)
+    plan = launch_plan(False, m, k, [n])
+    assert plan["kernel"] == "nf4_fwd8_kernel" and plan["rows_blocks"] == blocks
+    packed, qs, w = make_weight((n, k), seed=steps, device=device, nested=nested)
     x = randn16((m, k), seed=10 + blocks, device=device)
     (y,) = linear_forward(x, [dict(packed=packed, qs=qs)])
     assert_close(y, O.linear_ref(x.cpu().numpy(), w), what=f"{blocks} blocks, {steps} steps")
+
+
+@pytest.mark.parametrize("nested", [True, False])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("blocks", [2, 4, 7, 8, 9])
+def test_glu_few_steps(blocks, steps, nested, device, monkeypatch):
+    """Gate and up carry code books and code2 tables of their own (halves of LDS of their own)."""
+    from decik_amd.nf4 import glu_forward, launch_plan
+    from decik_amd.swiglu import swiglu_fwd
+
+    monkeypatch.setenv("DECIK_FWD_PLAN", f"{blocks},1,8")
+    m, n, k = ROWS[blocks] + 1, 136, 64 * steps
+    plan = launch_plan(False, m, k, [n, n], glu=True, nested=nested)
+    assert plan["kernel"] == "nf4_fwd8_kernel" and plan["rows_blocks"] == blocks
+    items, ws = [], []
+    for i in range(2):
+        p, q, w = make_weight((n, k), seed=steps + i, device=device, nested=nested)
+        if i == 1:
+            q.code = q.code.flip(0).contiguous()
+            if nested:
+                q.state2.code = q.state2.code.flip(0).contiguous()
+            w = O.dequant_nf4(oracle_state(p, q), nthreads=0)
+        items.append(dict(packed=p, qs=q))
+        ws.append(w)
+    x = randn16((m, k), seed=20 + blocks, device=device)
+    g, u, h = glu_forward(x, *items)
+    for out, w in zip((g, u), ws):
+        assert_close(out, O.linear_ref(x.cpu().numpy(), w), what=f"{blocks} blocks, {steps} steps")
+    assert torch.equal(h, swiglu_fwd(g, u))
 
 
 @pytest.mark.parametrize("n", [8, 56, 64, 72, 136, 200, 320])
@@ -65,12 +97,31 @@ def test_bwd_swiglu_large_tiles(m, n, k, plan, device, monkeypatch):
     assert torch.equal(dg3, dg) and torch.equal(du3, du)
 
 
+@pytest.mark.parametrize("nested", [True, False])
 @pytest.mark.parametrize("m", [9, 16, 17, 32])
+@pytest.mark.parametrize("n", [8200, 16392, 20488])  # row groups of 4, 5 and 6 tiles, one round, unsplit
 @pytest.mark.parametrize("k", [32, 128, 160, 1056])
-def test_small_m_last_items(m, k, device):
-    from decik_amd.nf4 import linear_forward
+def test_small_m_last_items(m, n, k, nested, device):
+    from decik_amd.nf4 import launch_plan, linear_forward
 
-    packed, qs, w = make_weight((2 ** 15 + 8, k), seed=k, device=device)
+    plan = launch_plan(False, m, k, [n])
+    assert plan["kernel"] == "nf4_skinny_kernel" and plan["splits"] == 1
+    packed, qs, w = make_weight((n, k), seed=k, device=device, nested=nested)
+    x = randn16((m, k), seed=m, device=device)
+    (y,) = linear_forward(x, [dict(packed=packed, qs=qs)])
+    assert_close(y, O.linear_ref(x.cpu().numpy(), w), what=f"m={m} n={n} k={k}")
+
+
+@pytest.mark.parametrize("m,kernel", [(9, "nf4_skinny_kernel"), (16, "nf4_skinny_kernel"),
+                                      (17, "nf4_fwd"), (32, "nf4_fwd")])
+@pytest.mark.parametrize("k", [32, 128, 160, 1056])
+def test_small_m_two_rounds(m, kernel, k, device):
+    """More than one row group a CU; past 16 rows the MFMA tiles."""
+    from decik_amd.nf4 import launch_plan, linear_forward
+
+    n = 2 ** 15 + 8
+    assert launch_plan(False, m, k, [n])["kernel"].startswith(kernel)
+    packed, qs, w = make_weight((n, k), seed=k, device=device)
     x = randn16((m, k), seed=m, device=device)
     (y,) = linear_forward(x, [dict(packed=packed, qs=qs)])
     assert_close(y, O.linear_ref(x.cpu().numpy(), w), what=f"m={m} k={k}")
