@@ -497,14 +497,16 @@ GemmPlan plan_skinny(int64_t m, int64_t k, const int64_t* ns, int ngroups, bool 
 
 // Forward launches of at most kSkinnyMaxM token rows without LoRA terms or the GLU epilogue run
 // the GEMV kernel (at most kGemvMaxM rows) or nf4_skinny_kernel, unless DECIK_FWD_PLAN forces an
-// MFMA plan. Measured on Qwen2.5-7B shapes: at one row the GEMV is faster on every shape (gate
-// 18 us against 25, q/o 10 against 16), and at two rows on all but the long contraction of down;
-// from 3 rows on the skinny kernel wins on all but small weights (gemv_requested; 7B gate at 8
-// rows: 28 us against 39 for the MFMA kernels). DECIK_SMALL_M = gemv / skinny forces one of them for launches both may take.
-// Past 16 rows (two 16-token blocks a work-group), weights of more row groups than CUs (even at
-// 6 tiles a group) go to the MFMA kernels: the skinny kernel's second round would hold few
-// work-groups (7B gate, 296 groups of 64 rows: 38.8 / 39.6 us at 24 / 32 rows against 34.2 /
-// 34.9 on 64-token MFMA tiles).
+// MFMA plan. Graph-replayed at one row the GEMV is the faster one on every shape measured (7B gate 13.0
+// us against 15.1, q/o 5.3 against 9.2, down 15.6 against 21.2, 1.5B gate 5.4 against 7.1), from two rows
+// on where gemv_requested says; the MFMA tiles are slower than either (7B gate at 8 / 16 / 32 rows 23.9 /
+// 24.5 / 25.6 against the small-M kernel's 16.7 / 17.5 / 21.6). DECIK_SMALL_M = gemv / skinny forces one
+// of the two for launches both may take. Past 16 rows (two 16-token blocks a work-group), weights of
+// more row groups than CUs (even at 6 tiles a group) go to the MFMA kernels: the small-M kernel's second
+// round holds few work-groups ([24592, 3584] at 17 / 24 / 32 rows 30.1 / 32.2 / 34.4 us against 31.3 /
+// 31.8 / 33.3 on 64-token MFMA tiles, [28672, 4096] 36.2 / 38.4 / 41.5 against 34.6 / 34.7 / 36.1, [24592,
+// 8192] 63.8 / 68.3 / 74.6 against 59.1 / 57.8 / 58.4; on short rows it would stay ahead: [32768, 1536]
+// 17.5 / 18.8 / 21.0 against 21.4 / 21.8 / 22.7).
 bool small_m_forward(int64_t m, bool glu, bool lora, const int64_t* ns, int ngroups) {
     if (glu || lora || m < 1 || m > kSkinnyMaxM) return false;
     const char* forced = std::getenv("DECIK_FWD_PLAN");
@@ -512,35 +514,47 @@ bool small_m_forward(int64_t m, bool glu, bool lora, const int64_t* ns, int ngro
     if (m > 16 && skinny_row_groups(ns, ngroups, skinny_row_tiles(ns, ngroups)) > num_cus()) return false;
     return true;
 }
-bool gemv_requested(int64_t m, int64_t k, const int64_t* ns, int ngroups) {
+// may_split: the small-M kernel may split this launch (the caller allows it and gave the workspace).
+bool gemv_requested(int64_t m, int64_t k, const int64_t* ns, int ngroups, bool may_split) {
     if (!gemv_fits(m, k)) return false;
     const char* v = std::getenv("DECIK_SMALL_M");
     if (v != nullptr && std::string(v) == "gemv") return true;
     if (v != nullptr && std::string(v) == "skinny") return false;
     if (m == 1) return true;
-    // Two rows: the GEMV's second dot product per weight costs in proportion to the weight, the
-    // small-M kernel hardly depends on the row count, so large launches take the small-M kernel.
-    // Graph-replayed at two rows, GEMV against small-M kernel: 7B gate 21.3-21.6 against 17.4 us
-    // (67.9M weights), 1.5B gate 8.1 against 8.8 (13.8M), 7B q/o 7.5 against 11.1 (12.8M); a
-    // long contraction also favours the small-M kernel's split (7B down, k = 18944: 23.7 against
-    // 35.1; the 1.5B down, k = 8960: 8.6 against 10.5 on the GEMV).
+    // Two rows and more: a GEMV work-group's further dot products per weight cost in proportion to the
+    // weight, the small-M kernel hardly depends on the row count, so large launches take the small-M
+    // kernel. All times graph-replayed, GEMV against small-M kernel, us. Lines that rest on the latter's
+    // split hold only where it may split: unsplit, few row groups are a long chain in a few work-groups.
     int64_t weights = 0;
     for (int g = 0; g < ngroups; ++g) weights += ns[g] * k;
-    // Long rows at two rows: up to 2^24 weights the GEMV still wins ([256, 20480] 8.2 against
-    // 11.0 us, [1024, 16384] 9.0 against 11.7); the 7B down projection (67.9M) does not.
-    if (m == 2) return weights < (int64_t(1) << 25) && (k <= 12288 || weights <= (int64_t(1) << 24));
+    // Two rows: up to 2^24 weights 1.5B gate 6.3 against 7.2, 7B q/o 6.4 against 9.3, 1.5B down 7.6 against
+    // 9.6, [2048, 8192] 10.2 against 10.4, [1024, 16384] 8.6 against 10.6, [256, 20480] 7.7 against 9.9 (but
+    // [2304, 7168] 11.4 against 10.1, [11264, 1408] 7.4 against 6.9). Larger ones by how X of two rows and the
+    // weight rows fill the LDS: up to k = 5632 [5120, 5120] 10.6 against 12.4, [11008, 2048] 8.4 against 10.1,
+    // [5888, 5632] 11.0 against 14.2; then [4096, 6144] 14.4 against 12.2, [3456, 7168] 15.3 against 12.3,
+    // [3584, 8192] 15.9 against 13.7; from k = 8704 (eight-wave work-groups) [3200, 8704] 11.5 against 12.7,
+    // [2560, 10240] 11.4 against 13.4, [2048, 12288] 11.5 against 12.3, past 27 2^20 weights [3600, 9216] 15.4
+    // against 13.7. 7B gate 16.3 against 15.2, 7B down 34.3 against 21.4.
+    if (m == 2)
+        return weights <= (int64_t(1) << 24) || (weights < (int64_t(1) << 25) && k <= (may_split ? 5632 : 12288)) ||
+               (weights <= (int64_t(27) << 20) && k >= 8704 && k <= 12288);
     // 3-8 rows (a GEMV work-group computes 4; past 4 rows two work-groups share each weight row
-    // range): small weights, whose small-M launches are bound by their fixed cost (a split and
-    // its reduction launch). At 3-4 rows every weight of up to 2^24: graph-replayed, GEMV against
-    // small-M kernel, us: 7B q/o 9.3 against 11.2, 1.5B gate 8.6 against 8.9, 1.5B down [1536,
-    // 8960] 10.4-10.7 against 11.5, [2048, 8192] 10.1 against 12.3, [1024, 12288] 10.3-10.4
-    // against 10.9-11.0, [896, 4864] 7.9-8.1 against 8.9-9.0 ([3584, 8192], 2^24.8 weights: 17.7
-    // against 15.1-15.2). Past 4 rows, X of 4 rows must stay within 32 KB of LDS per work-group. Graph-replayed, GEMV against small-M kernel, us:
-    // 1.5B k/v 4.3-4.5 / 6.3 against 8.1 / 8.3 at 3-4 / 8 rows, 1.5B q/o 4.9-5.0 / 6.9 against
-    // 8.4-8.6, the 1.5B q/k/v launch 5.1-5.3 / 7.1 against 8.6-8.8, 7B k/v 5.2 against 9.2 at
-    // 3-4 rows (11.6 against 9.4 at 8: X of 8 rows 56 KB); larger weights lose (7B q/o 11.9
-    // against 11.0, 7B gate 26 against 18, at 3 rows).
-    if (m <= 4) return weights <= (int64_t(1) << 24);
+    // range): weights whose small-M launch is split, which costs it a reduction launch. One unsplit
+    // round of the small-M kernel is the faster one: at 3-4 rows 1.5B gate 8.0 against 7.2, [8256, 512]
+    // 5.3 against 5.0, [16384, 1024] 8.7 against 6.9, [12288, 512] 5.6 against 5.1 (7.5 against 5.2 at 6);
+    // two such rounds are not at 3-4 rows ([30720, 256] 7.0 against 7.5; 9.5 against 7.7 at 6).
+    const int64_t rgroups = skinny_row_groups(ns, ngroups, skinny_row_tiles(ns, ngroups)), cus = num_cus();
+    if (2 * rgroups > cus && (m > 4 || rgroups <= cus)) return false;
+    // 3-4 rows up to 2^24 weights: 7B q/o 8.6 against 9.4, 1.5B down 9.6-9.9 against 9.8, [2048, 8192] 9.4-9.6
+    // against 10.6, [4096, 4096] 8.6 against 10.3, [896, 4864] 7.9 against 8.0, 7B k/v 4.7 against 7.5, 1.5B
+    // q/o 5.0 against 7.6 ([3584, 8192] 17.3 against 13.8, [3072, 5632], 17.3M, 12.3 against 10.8). Past k =
+    // 8192 X of four rows leaves a CU one work-group, and from about 15 2^20 weights they make a second
+    // round: [1280, 12288] 10.1 against 10.5, [1400, 10240] 9.6 against 10.5, [1408, 11264] 16.7 against 10.3,
+    // [1360, 12288] 17.5 against 11.0, [1024, 16384] 25.7 against 10.7.
+    if (m <= 4) return weights <= (k <= 8192 || !may_split ? int64_t(1) << 24 : int64_t(15) << 20);
+    // Past 4 rows, X of 4 rows must stay within 32 KB of LDS per work-group: at 6-8 rows 1.5B q/o 5.6-5.7
+    // against 7.7, [4864, 896] 7.0 against 7.8, [2048, 2048] 6.2-6.4 against 8.0, 7B k/v 5.4 against 7.8; larger
+    // weights lose ([4096, 4096] 12.5 against 10.4, 1.5B gate 11.3 against 7.4).
     return weights < (int64_t(1) << 23) && 4 * k * 2 <= 32768;
 }
 
@@ -712,7 +726,7 @@ int dk_nf4_linear_plan(int backward, int64_t m, int64_t k, const int64_t* ns, in
             }
         }
         kernel = 3;  // nf4_bwd8_kernel
-    } else if (small_m_forward(m, glu, lora, ns, ngroups) && gemv_requested(m, k, ns, ngroups)) {
+    } else if (small_m_forward(m, glu, lora, ns, ngroups) && gemv_requested(m, k, ns, ngroups, !single)) {
         p = GemmPlan{};
         int64_t nrows = 0;
         for (int g = 0; g < ngroups; ++g) nrows += ns[g];
@@ -850,10 +864,13 @@ static int linear_fwd_impl(const std::string& name, const uint16_t* x, int64_t m
         a.ncols = (int32_t)ncols;
         if (ncols > INT32_MAX / 2) return fail(name + ": problem too large");
         const hipStream_t st = static_cast<hipStream_t>(stream);
-        if (gemv_requested(m, k, ns, ngroups)) return check_hip(launch_gemv(a, st), "dk_nf4_linear_fwd GEMV launch");
+        if (gemv_requested(m, k, ns, ngroups, true)) return check_hip(launch_gemv(a, st), "dk_nf4_linear_fwd GEMV launch");
         const GemmPlan p = plan_skinny(m, k, ns, ngroups, no_split);
         const int64_t need = workspace_bytes(p);
-        if (need > 0 && (workspace == nullptr || workspace_bytes_ < need || !aligned(workspace, 256)))
+        const bool have = need == 0 || (workspace != nullptr && workspace_bytes_ >= need && aligned(workspace, 256));
+        if ((no_split || !have) && gemv_requested(m, k, ns, ngroups, false))
+            return check_hip(launch_gemv(a, st), "dk_nf4_linear_fwd GEMV launch");
+        if (!have)
             return fail(name + ": workspace too small (need " + std::to_string(need) + " bytes)");
         const int rows = 16 * p.row_tiles;
         int rg = 0;

@@ -322,19 +322,19 @@ int dk_swiglu_bwd(const uint16_t* grad, const uint16_t* gate, const uint16_t* up
  * first launch). blocksize: the largest block size of the groups' weights.
  * out[0] = 32-token row blocks per tile, out[1] = waves per work-group, out[2] = contraction
  * splits, out[3] = kernel (0 nf4_fwd_kernel, 1 nf4_fwd8_kernel, 2 no longer returned (an
- * earlier input-gradient kernel), 3 nf4_bwd8_kernel, 4 nf4_gemv_kernel (forward launches of one
- * token row, two with fewer than 2^25 weights and k <= 12288 (any k up to 2^24 weights), 3-4
- * with at most 2^24 weights, 5-8 with fewer than 2^23 weights
- * and 8 k <= 32768, without LoRA terms; GLU launches of one token row, two with k >= 2048
- * and at most 2048 weight rows, 1024 past k = 6144), 5
- * nf4_skinny_kernel (forward launches of up to 32 token rows without LoRA terms otherwise, but past
- * 16 rows not for weights of more 96-row groups than the device has CUs; out[2] is then its
- * contraction splits), 6 nf4_skinny_glu_kernel (such GLU launches otherwise, but not where further
- * rounds of its work-groups would outlast the MFMA tiles, as at [28672, 4096] from 12 token rows on
- * or [20544, 2048] from 24)); DECIK_SMALL_M = gemv / skinny picks the GEMV or the other few-row kernel where
- * both may run. Host-only (no GPU call);
- * honours DECIK_FWD_PLAN / DECIK_BWD_PLAN / DECIK_SMALL_M like the launches. Returns 0, or nonzero
- * with dk_last_error() on bad arguments. */
+ * earlier input-gradient kernel), 3 nf4_bwd8_kernel, 4 nf4_gemv_kernel (forward launches without
+ * LoRA terms of one token row, and of 2 to 8 on smaller weights; GLU launches of one, and of two on
+ * small weights of long rows), 5 nf4_skinny_kernel (such forward launches of up to 32 token rows
+ * otherwise, but past 16 rows not for weights of more 96-row groups than the device has CUs; out[2] is
+ * then its contraction splits), 6 nf4_skinny_glu_kernel (such GLU launches otherwise, but not where
+ * further rounds of its work-groups would outlast the MFMA tiles, as at [28672, 4096] from 12 token
+ * rows on or [20544, 2048] from 24)). The lines between them are measured ones; DECIK_SMALL_M = gemv /
+ * skinny picks the GEMV or the other few-row kernel where both may run. Forward launches without LoRA
+ * terms of one token row, two with fewer than 2^25 weights and k <= 12288 (any k up to 2^24 weights),
+ * 3-4 with at most 2^24 weights and 5-8 with fewer than 2^23 weights and 8 k <= 32768 need no
+ * workspace: given one, some of them run split on nf4_skinny_kernel, else on the GEMV. Host-only (no
+ * GPU call); honours DECIK_FWD_PLAN / DECIK_BWD_PLAN / DECIK_SMALL_M like the launches. Returns 0, or
+ * nonzero with dk_last_error() on bad arguments. */
 #define DK_PLAN_GLU 1
 #define DK_PLAN_LORA 2
 #define DK_PLAN_NO_SPLIT 4

@@ -182,8 +182,8 @@ def test_launch_plans():
     # at most 32 token rows, no LoRA, no GLU epilogue: the small-M kernel, split along the
     # contraction only where the rows cannot fill the GPU
     assert launch_plan(False, 1, 3584, [18944])["kernel"] == "nf4_gemv_kernel"
-    # two rows: the GEMV below 2^25 weights (k <= 12288, any k up to 2^24 weights), the small-M
-    # kernel above (7B gate: 67.9M)
+    # two rows: the GEMV up to 2^24 weights, and by row length below 2^25 (test_few_row_plans), the
+    # small-M kernel above (7B gate: 67.9M)
     assert launch_plan(False, 2, 20480, [256])["kernel"] == "nf4_gemv_kernel"
     assert launch_plan(False, 2, 18944, [3584])["kernel"] == "nf4_skinny_kernel"
     assert launch_plan(False, 2, 3584, [18944])["kernel"] == "nf4_skinny_kernel"
@@ -223,7 +223,7 @@ def test_launch_plans():
     assert launch_plan(False, 6, 3584, [3584])["kernel"] == "nf4_skinny_kernel"  # 7B q/o
     assert launch_plan(False, 8, 3584, [512])["kernel"] == "nf4_gemv_kernel"  # 7B k/v, two token groups
     assert launch_plan(False, 5, 8960, [256])["kernel"] == "nf4_skinny_kernel"  # X of 4 rows: 70 KB
-    # 3-4 rows: weights up to 2^24 (1.5B down, 7B q/o), not larger
+    # 3-4 rows: weights up to 2^24 (1.5B down, 7B q/o), not larger (test_few_row_plans)
     assert launch_plan(False, 4, 8960, [1536])["kernel"] == "nf4_gemv_kernel"
     assert launch_plan(False, 3, 3584, [3584])["kernel"] == "nf4_gemv_kernel"
     assert launch_plan(False, 3, 8192, [3584])["kernel"] == "nf4_skinny_kernel"
@@ -337,6 +337,25 @@ def test_glu_plans_of_two_rows(n, k, gemv):
     assert launch_plan(False, 2, k, [n, n], glu=True, nested=True)["kernel"] == \
         ("nf4_gemv_kernel" if gemv else "nf4_skinny_glu_kernel")
     assert launch_plan(False, 1, k, [n, n], glu=True, nested=True)["kernel"] == "nf4_gemv_kernel"
+
+
+@pytest.mark.parametrize("m,n,k,kernel,unsplit", [
+    # two rows, past 2^24 weights: by the row length (fourth: where the small-M kernel may split, fifth: where not)
+    (2, 1024, 16384, "gemv", "gemv"), (2, 5120, 5120, "gemv", "gemv"), (2, 3456, 7168, "skinny", "gemv"),
+    (2, 3584, 8192, "skinny", "gemv"), (2, 2560, 10240, "gemv", "gemv"), (2, 3600, 9216, "skinny", "gemv"),
+    # 3-4 rows: one unsplit round of the small-M kernel; long rows past 15 2^20 weights
+    (3, 8960, 1536, "skinny", "skinny"), (4, 8256, 512, "skinny", "skinny"), (3, 30720, 256, "gemv", "gemv"),
+    (3, 8192, 1536, "gemv", "gemv"), (4, 2048, 8192, "gemv", "gemv"), (3, 1280, 12288, "gemv", "gemv"),
+    (3, 1360, 12288, "skinny", "gemv"), (4, 1024, 16384, "skinny", "gemv"),
+    # 5-8 rows: never one against an unsplit small-M launch
+    (6, 2048, 2048, "gemv", "gemv"), (6, 8256, 512, "skinny", "skinny"), (8, 30720, 256, "skinny", "skinny"),
+])
+def test_few_row_plans(m, n, k, kernel, unsplit):
+    """GEMV or small-M kernel at two to eight token rows, both sides of each line as measured."""
+    from decik_amd.nf4 import launch_plan
+
+    assert launch_plan(False, m, k, [n])["kernel"] == f"nf4_{kernel}_kernel"
+    assert launch_plan(False, m, k, [n], no_split=True)["kernel"] == f"nf4_{unsplit}_kernel"
 
 
 def test_no_bit_cast_of_vector_elements():

@@ -458,3 +458,28 @@ def test_mfma_launches_statistics_forms_same_bits(m, device, monkeypatch):
     assert len(as_stored) == len(cached) == 12
     for i, (t1, t2) in enumerate(zip(as_stored, cached)):
         assert torch.equal(t1, t2), i
+
+
+@pytest.mark.parametrize("m,n,k,runs", [(2, 2056, 8320, True), (3, 1024, 16384, True), (9, 1024, 16384, False)])
+def test_few_rows_without_a_workspace(m, n, k, runs, device):
+    """Launches that the small-M kernel would split run on the GEMV where no workspace is given and it
+    takes launches of that size; larger ones are refused."""
+    from decik_amd._lib import LinearFwdGroup, lib, ptr, stream_of, weight_desc
+    from decik_amd.nf4 import launch_plan, linear_forward
+
+    assert launch_plan(False, m, k, [n])["kernel"] == "nf4_skinny_kernel" and launch_plan(False, m, k, [n])["splits"] > 1
+    packed, qs, w16 = make_weight((n, k), seed=n, device=device)
+    x = randn16((m, k), seed=m, device=device)
+    y = torch.full((m, n), 7.0, dtype=torch.float16, device=device)
+    groups = (LinearFwdGroup * 1)()
+    groups[0].w, keep = weight_desc(packed, qs, device)
+    groups[0].y, groups[0].ldy = y.data_ptr(), n
+    rc = lib().dk_nf4_linear_fwd(ptr(x), m, k, k, groups, 1, 0, None, 0, stream_of(device))
+    assert (rc == 0) == runs
+    if not runs:
+        assert b"workspace too small" in lib().dk_last_error()
+        return
+    ref = O.linear_ref(x.cpu().numpy(), w16)
+    assert_close(y, ref, what=f"m={m} without a workspace")
+    assert_close(linear_forward(x, [dict(packed=packed, qs=qs)])[0], ref, what=f"m={m}")
+    del keep

@@ -88,7 +88,7 @@ def test_random_small_m_forward(m, n, k, nested, bs, seed, device, monkeypatch):
     monkeypatch.setenv("DECIK_SMALL_M", "gemv")  # whether the GEMV can take the launch at all
     fits = launch_plan(False, m, k, [n], blocksize=bs)["kernel"] == "nf4_gemv_kernel"
     monkeypatch.delenv("DECIK_SMALL_M")
-    w = n * k
+    w = n * k  # at these sizes; the whole rule: test_abi.py, test_few_row_plans
     if m == 1 or (m == 2 and fits and w < 2 ** 25 and (k <= 12288 or w <= 2 ** 24)):
         assert kernel == "nf4_gemv_kernel"
     elif 3 <= m <= 4 and fits and w <= 2 ** 24:
