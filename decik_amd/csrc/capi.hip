@@ -158,7 +158,9 @@ int pad8(int g) { return (g + 7) & ~7; }
 //     else faster (one work-group per CU)
 //   + the split-K cost, proportional to the fp32 partial tiles written and read back.
 // Resident work-groups per CU and the step times are per-variant constants measured on MI355X
-// (Qwen2.5-1.5B MLP launches at M = 830).
+// (Qwen2.5-1.5B MLP launches at M = 830). The eight-wave kernels' steps have become 2-12% shorter since
+// (input gradients up to 20%), unevenly by tile; only the SwiGLU launches were fitted again to them
+// (kSwigluRoundUs).
 struct VariantCost {
     int rows_blocks;   // kernel template argument: token rows per tile / 32
     int waves;         // work-group waves (backward: 64 output columns each)
@@ -345,7 +347,7 @@ GemmPlan plan_fwd_compute(int64_t m, int64_t k, const int64_t* ns, int ngroups, 
     return p;
 }
 
-// swiglu: the SwiGLU epilogue of dk_nf4_linear_bwd_swiglu (never split; the variants that have it).
+// swiglu: the SwiGLU epilogue of dk_nf4_linear_bwd_swiglu (never split).
 // max_partial_bytes: the split-K partial slabs must fit in that many bytes.
 GemmPlan plan_bwd_compute(int64_t m, int64_t k, const int64_t* ns, int ngroups, bool swiglu, bool no_split,
                           int64_t max_partial_bytes) {
@@ -355,8 +357,9 @@ GemmPlan plan_bwd_compute(int64_t m, int64_t k, const int64_t* ns, int ngroups, 
     const int nv = kNumBwdVariants;
     no_split = no_split || swiglu;
     const VariantCost* v = plan_override("DECIK_BWD_PLAN", kBwdVariants, nv, p.steps, &p.splits);
-    // the SwiGLU epilogue never splits: on its larger tiles a forced plan with splits does not apply (on
-    // the smaller ones the splits alone are dropped)
+    // the SwiGLU epilogue never splits: of a forced plan with splits the smaller tiles drop the splits
+    // alone, while on the larger ones it does not apply (a plan forced for the split launches of a step
+    // left its SwiGLU launch to the planner before those tiles had the epilogue, and still does)
     if (v != nullptr && swiglu && v->rows_blocks > 4 && p.splits > 1) v = nullptr;
     if (v != nullptr && no_split) p.splits = 1;
     if (v != nullptr && p.splits > 1 && (double)p.splits * m * k * 4.0 > (double)max_partial_bytes) v = nullptr;
@@ -591,10 +594,11 @@ GluSmallM glu_small_m(int64_t m, int64_t k, int64_t n, bool lora) {
     // The small-M GLU kernel's work-groups take 16 * row_tiles rows of both weights. Beside its row tiles'
     // unpacking a work-group reads X once, which costs as much as 0.6 + 0.08 m row tiles, and a CU works
     // off its share of the work-groups: the row tiles with the least such work on the busiest CU, of
-    // those the most. Graph-replayed, us for 1 .. 5 tiles: 7B at 16 rows 55.7 / 43.3 / 38.0 / 43.8 / 28.7,
-    // at 32 97.2 / 69.2 / 55.8 / 61.6 / 38.2; 1.5B at 16 rows 15.4 / 13.8 / 10.6 / 12.1 / 13.9, at 32 27.3 /
-    // 22.7 / 14.7 / 15.9 / 18.7; [28672, 4096] at 16 rows 93.4 / 70.1 / 68.6 / 56.3 / 65.6 (by rows on the
-    // busiest CU alone one tile, the slowest, would win: 112 rows in seven work-groups).
+    // those the most. Graph-replayed (weight copies past the Infinity Cache), us for 1 .. 5 tiles: 7B at
+    // 16 rows 55.7 / 43.3 / 38.0 / 43.8 / 28.7, at 32 97.2 / 69.2 / 55.8 / 61.6 / 38.2; 1.5B at 16 rows 15.4 /
+    // 13.8 / 10.6 / 12.1 / 13.9, at 32 27.3 / 22.7 / 14.7 / 15.9 / 18.7; [28672, 4096] at 16 rows 93.4 / 70.1 /
+    // 68.6 / 56.3 / 65.6 (by rows on the busiest CU alone one tile, the slowest, would win: 112 rows in
+    // seven work-groups).
     const int64_t cus = num_cus();
     int64_t work = INT64_MAX;
     for (int rt = 1; rt <= 5; ++rt) {

@@ -178,7 +178,7 @@ hipError_t launch_skinny(const FwdArgs& a, int row_tiles, int grid, hipStream_t 
 // Gate and up with SwiGLU (no LoRA terms): nf4_skinny_glu_kernel, grid work-groups of 16 * row_tiles
 // (1 to 5) rows of both weights, no split
 hipError_t launch_skinny_glu(const FwdArgs& a, int row_tiles, int grid, hipStream_t s);
-// 8-wave forward kernel (32 weight rows x 32*mb tokens per wave), mb = 8 or 9
+// 8-wave forward kernel (32 weight rows x 32*mb tokens per wave), mb = 2, 4, 7, 8 or 9
 hipError_t launch_fwd8(const FwdArgs& a, int mb, int grid, hipStream_t s);
 // 8-wave input-gradient kernel (32 output columns x 32*mb tokens per wave), mb = 2, 4, 7 or 8
 hipError_t launch_bwd8(const BwdArgs& a, int mb, int grid, hipStream_t s);

@@ -338,7 +338,8 @@ __global__ __launch_bounds__(kB8Threads, 1) void nf4_bwd8_kernel(const BwdArgs a
         };
 
         // Ring buffers: step t uses dY buffer rd0 (byte offset in the dY ring), weight slot rw0
-        // and scale table si0; step t + 1 uses rd1 / rw1 / 1 - si0; step t + 3 reuses step t's.
+        // and scale table si0; step t + 1 uses rd1 / rw1 / 1 - si0. Step t + 3 reuses step t's weight slot
+        // and dY buffer, or with four dY buffers step t - 1's.
         int rd0 = 0, rw0 = 0, rd1 = DBUF, rw1 = kB8WSlot, si0 = 0;
         // Prologue: three steps in flight; wait for the first.
         load_step(t0, 0, 0, true);

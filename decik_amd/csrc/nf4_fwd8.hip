@@ -16,7 +16,7 @@
 //
 // Per wave and 64-wide step: one 16-byte packed load per lane (row arow_to_n(l32), k half
 // g = lane / 32) and the row's block statistics, through a per-wave LDS ring three steps deep;
-// the X tile through a shared ring three steps deep (buffer_load ... lds). Slice j (16 of k) =
+// the X tile through a shared ring three steps deep, four with MB = 2, 4 (buffer_load ... lds). Slice j (16 of k) =
 // one unpacked dword of 8 weights (A operand) x MB X fragments (B operands). The loop is
 // software-pipelined one slice ahead (its LDS reads two with MB = 2, 4): between the MFMAs of slice j
 // the wave refills each X fragment register right after its MFMA has read it and unpacks slice j + 1

@@ -123,9 +123,11 @@ __global__ __launch_bounds__(kSkThreads) void nf4_skinny_kernel(const FwdArgs a)
     // are read while the one before is packed (the scheduling barriers keep that order: left to
     // itself the compiler waits for each item's four reads as soon as they are issued), and one wait
     // covers the four. Two waves a SIMD issue an instruction every 4 to 5 cycles between them, so it
-    // is the instructions per item that count, 34 before and 24 now. 7B at 16 rows: gate and up in
-    // one launch 28.3 -> 25.3 us, q/k/v 8.7 -> 7.8; reading two items ahead was no faster, nor was a code book with
-    // one copy per pair of LDS banks, which takes the bank conflicts out of every read (26.5 -> 28.2).
+    // is the instructions per item that count, 34 before and 24 now. At 16 rows: 7B gate 18.1 -> 17.4 us,
+    // down 25.4 -> 23.0, q/k/v 8.7 -> 7.8, 1.5B gate 9.1 -> 8.2. Reading two items ahead was no faster, nor
+    // was a code book with one copy per pair of LDS banks, which takes the bank conflicts out of every
+    // read (7B gate and up in one launch of a form this kernel had: 26.5 -> 28.2). The small-M GLU kernel
+    // has the same loop over its items: what changes here is to be tried there.
     auto compute = [&](Step& st) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < RT; ++r) {

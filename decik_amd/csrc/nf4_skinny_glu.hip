@@ -11,7 +11,8 @@
 // rows of each weight, which a 7B MLP has 395 of for 256 CUs; and its 28 super-steps left half the
 // waves idle in the last of four rounds. Graph-replayed, gate+up, us: 7B at 3 / 16 / 32 rows 25.4 /
 // 25.9 / 43.4 -> 22.6 / 26.2 / 33.9, 1.5B 10.0 / 11.2 / 13.9 -> 8.9 / 10.5 / 14.0 (4 rows the first),
-// [13824, 5120] at 16 rows 31.2 -> 30.1, [4864, 896] 8.0 -> 5.8. At 16 rows of 7B the unpacking (24
+// [13824, 5120] at 16 rows 31.2 -> 30.1, [4864, 896] 8.0 -> 5.8. Its launches' row tiles and the
+// line to the MFMA tiles: glu_small_m in capi.hip. At 16 rows of 7B the unpacking (24
 // instructions per 8 weights a lane, an instruction every 4 to 5 cycles a SIMD) takes about two
 // thirds of the time, the loads alone the same.
 //

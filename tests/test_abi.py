@@ -167,15 +167,14 @@ def test_workspace_sizes():
 
 def test_launch_plans():
     """dk_nf4_linear_plan (host-only): the eight-wave input-gradient kernel serves the MLP's
-    gate/up input gradient at M = 830; SwiGLU-epilogue launches never split and use at most 4
-    token blocks; the fused GLU forward never splits; forced plans apply only where
-    their kernel may run; bad arguments are reported."""
+    gate/up input gradient at M = 830; SwiGLU-epilogue launches and the fused GLU forward never
+    split; forced plans apply only where their kernel may run; bad arguments are reported."""
     from decik_amd import _lib
     from decik_amd.nf4 import launch_plan
 
     gu = launch_plan(True, 830, 1536, [8960, 8960])
     assert gu["kernel"] == "nf4_bwd8_kernel" and gu["splits"] > 1
-    # the SwiGLU epilogue: never split, and only with at most 4 token blocks
+    # the SwiGLU epilogue: never split; one round of 128-token tiles here
     sw = launch_plan(True, 830, 8960, [1536], glu=True)
     assert sw["splits"] == 1
     assert sw["kernel"] == "nf4_bwd8_kernel" and sw["rows_blocks"] <= 4
@@ -279,7 +278,7 @@ def test_launch_plans():
         os.environ["DECIK_BWD_PLAN"] = "8,3,8"
         assert launch_plan(True, 830, 1536, [8960]) == dict(rows_blocks=8, waves=8, splits=3,
                                                              kernel="nf4_bwd8_kernel", launches=1, splits_second=0)
-        # no SwiGLU epilogue with 8 token blocks: the forced plan does not apply
+        # a forced plan with splits does not apply to the SwiGLU epilogue's larger tiles
         assert launch_plan(True, 830, 1536, [8960], glu=True)["rows_blocks"] != 8
         # variants that spilled registers are not offered: a forced plan naming one is ignored
         os.environ["DECIK_BWD_PLAN"] = "9,3,8"
