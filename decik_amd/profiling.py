@@ -12,9 +12,9 @@ This module reduces them to short markdown tables (or, for the traffic of one la
 `trace`: rocprofv3's own per-kernel totals, then every matching kernel by launch shape (grid):
 launches, median / mean / min duration, VGPRs, LDS. `counters`: per kernel and grid the mean of
 each counter over its dispatches and the usual ratios (VALU and LDS instructions per MFMA, MFMA
-busy share, wait share). `traffic`: HBM bytes per dispatch of the launch matched by RE (its most
-frequent kernel and grid, plus the split-K reduction dispatched right after it) from FETCH_SIZE
-and WRITE_SIZE, each scaled by what the counter reads for the fp32 -> fp16 conversion of 128 Mi
+busy share, wait share, LDS busy and bank-conflict shares, the clock of launches over 200 us).
+`traffic`: HBM bytes per dispatch of the launch matched by RE (its most frequent kernel and grid,
+plus the split-K reduction dispatched right after it) from FETCH_SIZE and WRITE_SIZE, each scaled by what the counter reads for the fp32 -> fp16 conversion of 128 Mi
 values that bench.py --copy-probe runs (512 MiB read, 256 MiB written). `traffic-table`: the same
 scaled bytes for every matching kernel and grid of several pass pairs, as a markdown table.
 """
@@ -80,6 +80,11 @@ def _counter_means(rows, match):
         if key not in acc:
             order.append(key)
         acc[key][r["Counter_Name"]].append(float(r["Counter_Value"]))
+        if r["Counter_Name"] == "GRBM_GUI_ACTIVE" and r.get("End_Timestamp"):
+            ns = int(r["End_Timestamp"]) - int(r["Start_Timestamp"])
+            acc[key]["duration us"].append(ns / 1e3)
+            if ns > 200e3:  # GRBM_GUI_ACTIVE also counts some 10 us around a launch
+                acc[key]["clock GHz"].append(float(r["Counter_Value"]) / 8 / ns)
     return order, {k: {c: statistics.fmean(v) for c, v in d.items()} for k, d in acc.items()}
 
 
@@ -97,9 +102,13 @@ def counter_summary(run_dirs_prefixes, title, commands, match=r"dk::"):
                                         "summed over the whole device.", ""]
     ratio_cols = [("VALU/MFMA", "SQ_INSTS_VALU", "SQ_INSTS_MFMA"), ("LDS/MFMA", "SQ_INSTS_LDS", "SQ_INSTS_MFMA"),
                   ("MFMA busy / SIMD-cycles", "SQ_VALU_MFMA_BUSY_CYCLES", None),
-                  ("wait / wave-cycles", "SQ_WAIT_INST_ANY", "SQ_WAVE_CYCLES")]
-    out += ["| kernel | grid | " + " | ".join(c[0] for c in ratio_cols) + " |",
-            "|---|---:|" + "---:|" * len(ratio_cols)]
+                  ("wait / wave-cycles", "SQ_WAIT_INST_ANY", "SQ_WAVE_CYCLES"),
+                  # of the time the launch has waves: SQ_BUSY_CYCLES (summed over 32 shader engines) / 32 x 256 CUs
+                  ("LDS busy", "SQ_LDS_IDX_ACTIVE", "SQ_BUSY_CYCLES"),
+                  ("bank conflicts / LDS busy", "SQ_LDS_BANK_CONFLICT", "SQ_LDS_IDX_ACTIVE")]
+    timed = ("duration us", "clock GHz")  # under the counters, each dispatch on its own
+    heads = [c[0] for c in ratio_cols] + list(timed)
+    out += ["| kernel | grid | " + " | ".join(heads) + " |", "|---|---:|" + "---:|" * len(heads)]
     for key in order:
         m = means[key]
         cells = []
@@ -110,9 +119,11 @@ def counter_summary(run_dirs_prefixes, title, commands, match=r"dk::"):
                 # SIMD-cycles of the dispatch: GRBM_GUI_ACTIVE (summed over the 8 XCDs) / 8 x 1024 SIMDs
                 cells.append(f"{m[num] / (m['GRBM_GUI_ACTIVE'] / 8 * 1024):.3f}" if "GRBM_GUI_ACTIVE" in m else "-")
             else:
-                cells.append(f"{m[num] / m[den]:.2f}" if m.get(den) else "-")
+                scale = 8 if den == "SQ_BUSY_CYCLES" else 1
+                cells.append(f"{m[num] / m[den] / scale:.2f}" if m.get(den) else "-")
+        cells += [f"{m[c]:.2f}" if c in m else "-" for c in timed]
         out.append(f"| `{_short(key[0], 60)}` | {key[1]} | " + " | ".join(cells) + " |")
-    names = sorted({c for m in means.values() for c in m})
+    names = sorted({c for m in means.values() for c in m} - set(timed))
     out += ["", "Raw means per dispatch:", "", "| counter | " + " | ".join(f"`{_short(k[0], 40)}` {k[1]}" for k in order) + " |",
             "|---|" + "---:|" * len(order)]
     for c in names:
