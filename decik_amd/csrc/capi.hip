@@ -713,8 +713,17 @@ int dk_nf4_linear_plan(int backward, int64_t m, int64_t k, const int64_t* ns, in
     if (ngroups < 1 || ngroups > kMaxGroups || ns == nullptr || out == nullptr || m <= 0 || k <= 0 ||
         blocksize < 32 || log2_exact(blocksize) < 0)
         return fail("dk_nf4_linear_plan: bad arguments");
-    const bool glu = (flags & DK_PLAN_GLU) != 0, lora = (flags & DK_PLAN_LORA) != 0;
-    const bool single = (flags & DK_PLAN_NO_SPLIT) != 0;
+    const bool lora = (flags & DK_PLAN_LORA) != 0;
+    bool glu = (flags & DK_PLAN_GLU) != 0, single = (flags & DK_PLAN_NO_SPLIT) != 0;
+    const GluSmallM gs = !backward && glu && ngroups == 2 && ns[0] == ns[1] && blocksize >= 64 && k % 64 == 0
+                             ? glu_small_m(m, k, ns[0], lora)
+                             : GluSmallM{};
+    // gate and up that dk_nf4_glu_fwd runs as a grouped launch without a workspace
+    if (!backward && glu && gs.kernel == GluSmallM::kMfma &&
+        (blocksize < 64 || k % 64 != 0 || ((flags & DK_PLAN_NESTED) != 0 && k % blocksize != 0))) {
+        glu = false;
+        single = true;
+    }
     GemmPlan p;
     int kernel;
     int launches = 1, splits_b = 0;
@@ -740,10 +749,7 @@ int dk_nf4_linear_plan(int backward, int64_t m, int64_t k, const int64_t* ns, in
     } else if (small_m_forward(m, glu, lora, ns, ngroups)) {
         p = plan_skinny(m, k, ns, ngroups, single);
         kernel = 5;  // nf4_skinny_kernel
-    } else if (const GluSmallM gs = glu && ngroups == 2 && ns[0] == ns[1] && blocksize >= 64 && k % 64 == 0
-                                        ? glu_small_m(m, k, ns[0], lora)
-                                        : GluSmallM{};
-               gs.kernel != GluSmallM::kMfma) {
+    } else if (gs.kernel != GluSmallM::kMfma) {
         p = GemmPlan{};
         p.mt = gs.kernel == GluSmallM::kSkinny ? (m <= 16 ? 1 : 2) : 0;
         p.waves = 8;
@@ -1016,15 +1022,19 @@ int dk_nf4_glu_fwd(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
     const int64_t n = wg.n;
     if (m > 0 && (!aligned(h, 16) || ldh < n || (ldh % 8) != 0))
         return fail("dk_nf4_glu_fwd: h must be 16-byte aligned with ldh >= n, ldh % 8 == 0");
-    const bool fused = wg.nested == wu.nested && wg.blocksize == wu.blocksize && wg.blocksize >= 64 &&
-                       k % 64 == 0;
+    bool fused = wg.nested == wu.nested && wg.blocksize == wu.blocksize && wg.blocksize >= 64 && k % 64 == 0;
+    // nested blocks that straddle rows: of the tiled kernels only the four-wave one may run, and its GLU
+    // waves read one weight's nested statistics
+    if (fused && wg.nested && k % wg.blocksize != 0)
+        fused = glu_small_m(m, k, n, groups[0].lora_u != nullptr || groups[1].lora_u != nullptr).kernel != GluSmallM::kMfma;
     if (fused)
         return linear_fwd_impl("dk_nf4_glu_fwd", x, m, k, ldx, groups, 2, lora_rank, nullptr, 0, stream,
                                h, ldh, true);
     // other statistics: gate and up by the grouped launch (one pass), then the SwiGLU kernel
     if (m > 0 && (groups[0].y == nullptr || groups[1].y == nullptr || groups[0].ldy != n ||
                   groups[1].ldy != n || ldh != n))
-        return fail("dk_nf4_glu_fwd: narrow-block or mixed-statistics weights need gate and up outputs, all rows contiguous");
+        return fail("dk_nf4_glu_fwd: narrow-block, row-straddling nested or mixed-statistics weights need gate and up outputs, "
+                    "all rows contiguous");
     if (linear_fwd_impl("dk_nf4_glu_fwd", x, m, k, ldx, groups, 2, lora_rank, nullptr, 0, stream, nullptr,
                         0, true))
         return 1;

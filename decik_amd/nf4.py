@@ -323,27 +323,37 @@ def _fwd_group(g, it, dev, keep):
     keep += [bias, u, b]
 
 
+def _glu_one_launch(gate_qs, up_qs, k):
+    """Whether dk_nf4_glu_fwd takes these weights in one launch at any row count (else it needs the
+    gate and up outputs)."""
+    bs = int(gate_qs.blocksize)
+    return (gate_qs.nested == up_qs.nested and bs == int(up_qs.blocksize) and bs >= 64 and k % 64 == 0
+            and (not gate_qs.nested or k % bs == 0))
+
+
 def glu_forward(x16, gate, up, keep_gate_up=True, lora_rank=0):
     """(gate_out, up_out, h) with h = silu(gate_out) * up_out, one launch (dk_nf4_glu_fwd).
 
     gate / up: dicts as for linear_forward (packed, qs, optional bias, lora_u, lora_b,
-    lora_scale). keep_gate_up=False skips storing gate_out and up_out (returned as None)."""
+    lora_scale). keep_gate_up=False skips storing gate_out and up_out (returned as None); weights
+    that the entry runs as two launches have them stored all the same, for the call's duration."""
     dev = x16.device
     x2 = _rows(x16)
     m, k = x2.shape
     n = int(gate["qs"].shape[0])
     groups = (LinearFwdGroup * 2)()
     keep, outs = [x2], []
+    stored = keep_gate_up or not _glu_one_launch(gate["qs"], up["qs"], k)
     for g, it in enumerate((gate, up)):
         _fwd_group(groups[g], it, dev, keep)
-        out = torch.empty((m, n), dtype=torch.float16, device=dev) if keep_gate_up else None
+        out = torch.empty((m, n), dtype=torch.float16, device=dev) if stored else None
         groups[g].y = None if out is None else out.data_ptr()
         groups[g].ldy = n
         outs.append(out)
     h = torch.empty((m, n), dtype=torch.float16, device=dev)
     check(lib().dk_nf4_glu_fwd(ptr(x2), m, k, x2.stride(0), groups, int(lora_rank), ptr(h), n,
                                stream_of(dev)))
-    return outs[0], outs[1], h
+    return (outs[0], outs[1], h) if keep_gate_up else (None, None, h)
 
 
 def linear_backward_swiglu(item, gate, up, out=None, lora_rank=0):

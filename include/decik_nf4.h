@@ -164,8 +164,8 @@ int dk_nf4_linear_rope_fwd(const uint16_t* x, int64_t m, int64_t k, int64_t ldx,
  * token row that of dk_nf4_linear_fwd, otherwise one of three by row count (GEMV, small-M kernel,
  * MFMA tiles) -- so a few of them round to the other neighbouring fp16 value than in
  * dk_nf4_linear_fwd, or in a call of another row count. One launch when gate and up have the same
- * statistics kind (both plain or both nested, as bitsandbytes stores them), blocksize >= 64 and
- * k % 64 == 0; then groups[i].y may be NULL (not stored). Other weights run as the grouped launch
+ * statistics kind (both plain or both nested, as bitsandbytes stores them), blocksize >= 64,
+ * k % 64 == 0 and, of nested statistics, k % blocksize == 0 (or the few-row forms run); then groups[i].y may be NULL (not stored). Other weights run as the grouped launch
  * then the SwiGLU kernel and need both y, with rows contiguous (ldy = ldh = n). Up to 32 token rows
  * without LoRA terms run the GLU forms of the GEMV and the small-M kernel, but from 12 rows on not
  * for every weight of more than 20480 rows (dk_nf4_linear_plan). No workspace. */
@@ -319,7 +319,7 @@ int dk_swiglu_bwd(const uint16_t* grad, const uint16_t* gate, const uint16_t* up
  * nested statistics), DK_PLAN_PARTS (out holds 6 values: out[4] = GEMM launches of the call, 2
  * when an input gradient whose tiles overrun whole rounds of CUs runs its left-over columns as a
  * second launch, and out[5] = that launch's contraction splits; out[0..3] then describe the
- * first launch). blocksize: the largest block size of the groups' weights.
+ * first launch). Of gate and up that dk_nf4_glu_fwd runs as two launches, the first. blocksize: the largest block size of the groups' weights.
  * out[0] = 32-token row blocks per tile, out[1] = waves per work-group, out[2] = contraction
  * splits, out[3] = kernel (0 nf4_fwd_kernel, 1 nf4_fwd8_kernel, 2 no longer returned (an
  * earlier input-gradient kernel), 3 nf4_bwd8_kernel, 4 nf4_gemv_kernel (forward launches without

@@ -357,6 +357,19 @@ def test_few_row_plans(m, n, k, kernel, unsplit):
     assert launch_plan(False, m, k, [n], no_split=True)["kernel"] == f"nf4_{unsplit}_kernel"
 
 
+@pytest.mark.parametrize("m,k,blocksize,nested", [(830, 1600, 128, True), (830, 1536, 32, True),
+                                                  (20, 1536, 32, False), (830, 1568, 64, False)])
+def test_glu_plans_of_two_launches(m, k, blocksize, nested):
+    """Gate and up whose statistics no GLU tile reads (blocks under 64, steps across blocks, nested
+    blocks across rows) are planned as the grouped launch, unsplit."""
+    from decik_amd.nf4 import launch_plan
+
+    glu = launch_plan(False, m, k, [8960, 8960], glu=True, nested=nested, blocksize=blocksize)
+    assert glu == launch_plan(False, m, k, [8960, 8960], no_split=True, blocksize=blocksize) and glu["splits"] == 1
+    assert launch_plan(False, 20, 1600, [8960, 8960], glu=True, nested=True, blocksize=128)["kernel"] == \
+        "nf4_skinny_glu_kernel"
+
+
 def test_no_bit_cast_of_vector_elements():
     """hipcc compiles __builtin_bit_cast(T, v[i]) of an ext_vector_type element as element 0
     whatever i is (found twice in this library); the kernels copy elements to scalars first.

@@ -125,6 +125,59 @@ def test_glu_forward_nested_statistics_one_launch(m, n, k, plan, device, monkeyp
     del keep, keep2
 
 
+@pytest.mark.parametrize("recompute", [True, False])
+@pytest.mark.parametrize("blocksize,hidden", [(128, 192), (32, 192), (64, 192)])
+@pytest.mark.parametrize("m", [5, 70])
+def test_mlp_where_gate_and_up_take_two_launches(m, blocksize, hidden, recompute, device):
+    """FusedMLP on nested blocks across rows and on narrow blocks, where the forward keeps no gate and
+    up for the backward: the same output and gradient as with them kept, and as the oracle's."""
+    from decik_amd.mlp import FusedMLP
+
+    inter = 256
+    packs = [make_weight(s, seed=120 + i, device=device, std=0.02 * (i + 1), blocksize=blocksize)
+             for i, s in enumerate(((inter, hidden), (inter, hidden), (hidden, inter)))]
+    x = randn16((m, hidden), seed=m, device=device).requires_grad_()
+    dy = randn16((m, hidden), seed=m + 1, device=device, std=1e-2)
+    args = [t for p, q, _ in packs for t in (p, q)]
+    y = FusedMLP.apply(x, *args, recompute)
+    (dx,) = torch.autograd.grad(y, x, dy)
+    xr = x.detach().double().cpu().requires_grad_()
+    wg, wu, wd = (torch.from_numpy(w).double() for _, _, w in packs)
+    yr = (torch.nn.functional.silu(xr @ wg.T) * (xr @ wu.T)) @ wd.T
+    (dxr,) = torch.autograd.grad(yr, xr, dy.double().cpu())
+    # the fp16 gate, up, hidden and gradient values between the products: four roundings of 2.1e-4 each
+    for out, ref in ((y, yr), (dx, dxr)):
+        assert float((out.double().cpu() - ref).detach().norm() / ref.detach().norm()) < 1e-3
+
+
+@pytest.mark.parametrize("keep", [True, False])
+@pytest.mark.parametrize("m,n,k,blocksize", [(1, 72, 192, 128), (20, 72, 192, 128), (33, 136, 192, 128),
+                                             (300, 264, 320, 256), (64, 128, 1600, 128)])
+def test_glu_forward_nested_blocks_across_rows(m, n, k, blocksize, keep, device):
+    """Nested statistics whose blocks straddle weight rows (k % blocksize != 0), where the eight-wave
+    kernel may not run: gate and up of different spread, each by its own statistics."""
+    from decik_amd.nf4 import glu_forward
+    from decik_amd.swiglu import swiglu_fwd
+
+    items, ws = [], []
+    for i, std in enumerate((0.02, 0.06)):
+        p, q, w = make_weight((n, k), seed=90 + i, device=device, std=std, blocksize=blocksize)
+        items.append(dict(packed=p, qs=q))
+        ws.append(w)
+    x = randn16((m, k), seed=m, device=device)
+    g, u, h = glu_forward(x, *items, keep_gate_up=keep)
+    xn = x.cpu().numpy()
+    refs = [O.linear_ref(xn, w, None) for w in ws]
+    if keep:
+        for out, ref in zip((g, u), refs):
+            assert_close(out, ref, what=f"{m}x{n}x{k}")
+        assert torch.equal(h, swiglu_fwd(g, u))
+    else:
+        assert g is None and u is None
+        full = glu_forward(x, *items)
+        assert torch.equal(h, full[2])
+
+
 def test_glu_forward_narrow_blocks_take_two_launches(device):
     """Weights of 32-element blocks run the grouped launch and the SwiGLU kernel; without gate/up
     outputs the entry refuses."""
