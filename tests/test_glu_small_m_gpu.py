@@ -100,3 +100,33 @@ def test_glu_few_rows_strided(m, n, device):
     check(lib().dk_nf4_glu_fwd(ptr(xw), m, k, k + pad, groups, 0, ptr(outs[2]), n + pad, stream_of(device)))
     for out, ref in zip(outs, want):
         assert torch.equal(out[:, :n], ref) and bool((out[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 264, 576), (2, 264, 2112), (3, 264, 576), (20, 264, 576)])
+@pytest.mark.parametrize("nested", [True, False])
+def test_glu_few_rows_optional_operands(m, n, k, nested, device):
+    """One output and one bias at a time, and token rows of infinities and NaN, which stay in their
+    rows (rows past m, the contraction's tail and weight rows past n read as zeros beside them)."""
+    from decik_amd._lib import LinearFwdGroup, check, lib, ptr, stream_of, weight_desc
+    from decik_amd.nf4 import glu_forward
+
+    items = [make_weight((n, k), seed=30 + i, device=device, nested=nested)[:2] for i in range(2)]
+    bias = randn16((n,), seed=9, device=device, std=0.2)
+    x = randn16((m, k), seed=m, device=device)
+    for which in range(2):
+        dicts = [dict(packed=p, qs=q, bias=bias if i == which else None) for i, (p, q) in enumerate(items)]
+        want = glu_forward(x, *dicts)
+        y, h = (torch.full((m, n), 7.0, dtype=torch.float16, device=device) for _ in range(2))
+        groups, keep = (LinearFwdGroup * 2)(), []
+        for i, (p, q) in enumerate(items):
+            groups[i].w, kp = weight_desc(p, q, device)
+            keep.append(kp)
+        groups[which].y, groups[which].ldy, groups[which].bias = y.data_ptr(), n, bias.data_ptr()
+        check(lib().dk_nf4_glu_fwd(ptr(x), m, k, k, groups, 0, ptr(h), n, stream_of(device)))
+        assert torch.equal(y, want[which]) and torch.equal(h, want[2])
+    for bad in (float("inf"), float("nan")):
+        xb = x.clone()
+        xb[m - 1] = bad
+        out = glu_forward(xb, *dicts)
+        for a, b in zip(out, want):
+            assert torch.equal(a[:m - 1], b[:m - 1]) and not bool(torch.isfinite(a[m - 1]).any())
